@@ -651,9 +651,10 @@ static int block_forward_impl(const brx_layer_desc* d, brx_pool* p, const void* 
     void* ws = nullptr;
     size_t ws_bytes = 0;
     if (scratch_ws) {
-        if (route_b + fwd_b > scratch_bytes)
+        const size_t min_b = route_b + (decode ? fwd_b : prefill_workspace_min(a));
+        if (min_b > scratch_bytes)
             return fail(BRX_EINVAL, "this call needs %zu bytes of scratch, the no-alloc scratch holds %zu "
-                        "(T=%d); use brx_moe_block_forward", route_b + fwd_b, scratch_bytes, T);
+                        "(T=%d); use brx_moe_block_forward", min_b, scratch_bytes, T);
         ws = scratch_ws;
         ws_bytes = scratch_bytes;
     } else {

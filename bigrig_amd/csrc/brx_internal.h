@@ -243,9 +243,11 @@ __device__ __forceinline__ float e2m1_f32(uint32_t c) {
 
 // e8m0 -> 2^(e-127) (NaN for 0xFF)
 __device__ __forceinline__ float e8m0_f32(uint32_t e) {
-    if (e == 255u) return __uint_as_float(0x7fc00000u);
-    if (e == 0u) return __uint_as_float(0x00400000u);  // 2^-127, subnormal in fp32
-    return __uint_as_float(e << 23);
+    // selects, not returns: those become branches that split a K loop's straight-line code
+    uint32_t b = e << 23;
+    b = e == 0u ? 0x00400000u : b;     // 2^-127, subnormal in fp32
+    b = e == 255u ? 0x7fc00000u : b;
+    return __uint_as_float(b);
 }
 
 // x * sigmoid(a x) = x / (1 + 2^(-a x log2(e))) with the hardware exp2 and reciprocal
@@ -651,6 +653,7 @@ hipError_t launch_decode(const FwdArgs& a, void* ws, int phases, hipStream_t s);
 hipError_t launch_decode_wide(const FwdArgs& a, void* ws, int phases, hipStream_t s);   // 2, 6, 8 bits
 hipError_t launch_prefill(const FwdArgs& a, void* ws, size_t ws_bytes, int phases, hipStream_t s);
 size_t prefill_workspace_bytes(const FwdArgs& a);
+size_t prefill_workspace_min(const FwdArgs& a);
 size_t decode_workspace_bytes(const FwdArgs& a);
 hipError_t launch_dequant(const brx_layer_desc& d, const Layout& L, const uint8_t* expert,
                           int proj, float* out, hipStream_t s);

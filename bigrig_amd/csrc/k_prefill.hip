@@ -32,7 +32,7 @@
 // all its N tiles.
 #include <type_traits>
 
-#include "brx_internal.h"
+#include "pf_common.h"
 
 namespace brx {
 namespace {
@@ -40,7 +40,6 @@ namespace {
 constexpr int kBM = 128;          // pairs per M tile
 constexpr int kBK = 64;           // K step
 constexpr int kThreads = 256;
-constexpr int kXcd = 8;
 
 // ------------------------------------------------------------------ bucketing
 // Pairs are read coalesced: in each pass of kBucketPass pairs, wave w takes the 1024 pairs
@@ -218,19 +217,6 @@ __global__ __launch_bounds__(kBucketThreads) void k_bucket(const int32_t* __rest
     }
 }
 
-__device__ __forceinline__ int pair_token(const FwdArgs& a, int pair) {
-    return pair < a.P ? pair_tok(a, pair) : pair - a.P;
-}
-
-__device__ __forceinline__ uint32_t pk_bf16(float lo, float hi) {
-    return __builtin_bit_cast(uint32_t, bf16x2_t{(__bf16)lo, (__bf16)hi});
-}
-
-// native vector (not HIP's uint4 struct, whose copies are memcpys that keep arrays of it in
-// scratch memory)
-typedef uint32_t u32x4_t __attribute__((ext_vector_type(4)));
-typedef uint32_t u32x3_t __attribute__((ext_vector_type(3)));
-
 // ------------------------------------------------------------------ grouped GEMM
 // One block = 256 threads = 4 waves, one wave per SIMD; the tile is MF * 16 rows (one M tile
 // of one expert, MF in {2, 4, 8} chosen by the tile's row count) by 256 columns, wave w owning
@@ -282,30 +268,6 @@ static_assert(kNS * kStage <= kRing, "the per-stage ring must fit");
 static_assert(kNS * (2 * 16 * kBK * 2 + kStS) + kBPairLds <= kRing, "a 32-row tile's ring and B staging must fit");
 static_assert(8 * 16 * (kBlockN + 8) * 2 <= kRing, "the widest output tile must fit in the ring");
 
-typedef __attribute__((address_space(3))) void* LDS_PTR;
-typedef uint32_t u32x2_t __attribute__((ext_vector_type(2)));
-
-// swizzle key of A tile row m: 16-byte chunk c of the row sits in slot c ^ a_key(m); rows
-// 2t and 2t + 1 share a 256-byte bank row, so keys (m >> 1) & 7 spread 16 consecutive rows
-// over 16 distinct bank groups
-__device__ __forceinline__ int a_key(int m) { return (m >> 1) & 7; }
-
-// waits for this wave's LDS accesses, then for every wave
-__device__ __forceinline__ void lds_barrier() {
-    asm volatile("s_waitcnt lgkmcnt(0)\n\ts_barrier" ::: "memory");
-}
-
-// waits until at most N of this wave's memory loads (copies into LDS and loads into registers)
-// are in flight, then for every wave. The wait is the builtin, so the compiler's own wait
-// placement knows which loads it covers and adds none for the registers it has made ready;
-// the barrier is inline asm with a memory clobber, so no LDS access moves across it.
-template <int N>
-__device__ __forceinline__ void dma_wait_barrier() {
-    static_assert(N >= 0 && N < 64, "vmcnt is 6 bits");
-    __builtin_amdgcn_s_waitcnt((N & 0xF) | (0x7 << 4) | (0xF << 8) | ((N >> 4) << 14));
-    asm volatile("s_barrier" ::: "memory");
-}
-
 // Copies into LDS a wave has issued after stage s + 1's when it waits for stage s + 1 at
 // iteration s (s of parity par): those of stages s + 2 .. s + ns - 2, nv0 for an even stage,
 // nv1 for an odd one.
@@ -315,73 +277,11 @@ constexpr int loads_after(int ns, int nv0, int nv1, int par) {
     return n;
 }
 
-__device__ __forceinline__ __amdgpu_buffer_rsrc_t make_rsrc(const void* p, uint32_t bytes) {
-    return __builtin_amdgcn_make_buffer_rsrc(const_cast<void*>(p), (short)0, (int)bytes, 0x00020000);
-}
-
-// Dequantize piece kk (8 weights, natural K order) of a lane's words `w` into a bf16x8 MFMA
-// operand.
-//   affine: w = s q + b with one fp32 rounding, then rounded to bf16 (v_cvt_pk_bf16_f32).
-//     Each code q is read as the fp16 subnormal q 2^-24 (the code alone in a 16-bit half, exact
-//     when widened to fp32: q < 1024) and v_fma_mix_f32 forms fma(q 2^-24, s 2^24, b): the
-//     product is exactly s q, so the result is the same fl(s q + b) as fmaf(s, q, b). `s24` is
-//     s 2^24 (exact for any scale below 2^104). piece_pair puts codes i and 4 + i in the two
-//     halves of one register, so a 4-bit piece costs 7 extractions, 8 fma_mix and 4 packs.
-//   MXFP4: the hardware converts two e2m1 codes with the e8m0 scale, exact in bf16.
-//   Unquantized bf16 weights are the operand as loaded.
-template <int MODE>
-__device__ __forceinline__ bf16x8_t dq8(const uint32_t* w, int kk, float s24, float b, float sc) {
-    uint32_t o[4];
-    if constexpr (kAffine<MODE>) {
-        float v[8];
-#pragma unroll
-        for (int i = 0; i < 4; ++i) {
-            // codes i (low half) and 4 + i (high half)
-            const uint32_t t = piece_pair<kBits<MODE>>(w, kk, i);
-            v[i] = __builtin_fmaf((float)__builtin_bit_cast(_Float16, (uint16_t)(t & 0xFFFFu)), s24, b);
-            v[4 + i] = __builtin_fmaf((float)__builtin_bit_cast(_Float16, (uint16_t)(t >> 16)), s24, b);
-        }
-#pragma unroll
-        for (int j = 0; j < 4; ++j) o[j] = pk_bf16(v[2 * j], v[2 * j + 1]);
-    } else if constexpr (MODE == kModeBf16) {
-        // unquantized: the piece is 8 bf16 weights, 4 words in natural K order
-#pragma unroll
-        for (int j = 0; j < 4; ++j) o[j] = w[4 * kk + j];
-    } else {
-        const uint32_t q = w[kk];
-        o[0] = __builtin_bit_cast(uint32_t, __builtin_amdgcn_cvt_scalef32_pk_bf16_fp4(q, sc, 0));
-        o[1] = __builtin_bit_cast(uint32_t, __builtin_amdgcn_cvt_scalef32_pk_bf16_fp4(q, sc, 1));
-        o[2] = __builtin_bit_cast(uint32_t, __builtin_amdgcn_cvt_scalef32_pk_bf16_fp4(q, sc, 2));
-        o[3] = __builtin_bit_cast(uint32_t, __builtin_amdgcn_cvt_scalef32_pk_bf16_fp4(q, sc, 3));
-    }
-    return __builtin_bit_cast(bf16x8_t, u32x4_t{o[0], o[1], o[2], o[3]});
-}
-
-// B words a lane holds per stage (half of a row's 64-code stage segment: 32 codes), and the
-// loads that bring them in (16-byte loads, plus one 8-byte load for 6 bits; one 8- or 12-byte
-// load for 2 and 3 bits; four 16-byte loads for bf16 weights).
-template <int MODE>
-constexpr int kBW = kBits<MODE>;
-template <int MODE>
-constexpr int kBLoads = kBits<MODE> == 16 ? 4 : kBits<MODE> >= 6 ? 2 : 1;
 // M tile height: 128 rows, or 64 for 6- and 8-bit codes and bf16 weights, whose B words (48, 64
 // and 128 registers over the ring) leave no room for the accumulators of a 128-row tile at two
 // blocks per CU
 template <int MODE>
 constexpr int kTileRows = kBits<MODE> >= 6 ? 64 : 128;
-
-// The activation of one output element with the rule fixed at compile time (act_apply's
-// arithmetic for that rule, so the same bits).
-template <int ACT>
-__device__ __forceinline__ float act_fixed(float g, float u, float alpha, float limit) {
-    if constexpr (ACT == BRX_ACT_SWIGLU) return silu_mul(g, u);
-    else if constexpr (ACT == BRX_ACT_SILU_MLP) return x_sigmoid(g, 1.0f);
-    else {
-        g = fminf(g, limit);
-        u = fminf(fmaxf(u, -limit), limit);
-        return x_sigmoid(g, alpha) * (u + 1.0f);
-    }
-}
 
 // The gate/up epilogue of one activation rule: act(gate + bias, up + bias) (or SiLU(fc1 + bias))
 // of every accumulator into the LDS tile T (row stride TS elements), NaN for an absent expert.
@@ -1119,14 +1019,14 @@ inline int tile_rows(int mode) {
     return mode == kModeAffine6 || mode == kModeAffine8 || mode == kModeBf16 ? 64 : kBM;
 }
 
-PfWs carve(const FwdArgs& a, void* ws) {
+PfWs carve(const FwdArgs& a, int tile, void* ws) {
     const int P = a.P;
     const int T_sh = a.auto_shared ? a.T : 0;
     const int P_ext = P + T_sh;
     const int E_ext = a.E + (a.shared ? 1 : 0);
     const int Imax = a.I > a.I_sh ? a.I : a.I_sh;
     // at most ceil(P_ext / BM) full tiles plus one partial tile per expert
-    const int BM = tile_rows(a.quant_mode);
+    const int BM = tile;
     const int mt_max = (P_ext + BM - 1) / BM + E_ext;
     PfWs w{};
     w.mt_pad = (mt_max + kXcd - 1) / kXcd * kXcd;
@@ -1177,7 +1077,26 @@ hipError_t launch_bucket(const int32_t* pexp, int P, int E, int E_ext, int T_sh,
 
 }  // namespace
 
-size_t prefill_workspace_bytes(const FwdArgs& a) { return carve(a, nullptr).bytes; }
+// The M tile height of a call whose tiles all go to the thin-tile GEMM (k_thin.hip), or 0 for
+// k_pf_gemm. The line is the mean number of pairs an expert: both kernels within 2% at 48 (777
+// tokens of 128 3-bit experts, 179 against 176 us), the thin one faster at 32 (512 tokens of 4-bit
+// experts, two layers: 272 against 290 us) and below.
+static int thin_rows(const FwdArgs& a) {
+    constexpr int kThinPairs = 40;
+    const int64_t P_ext = a.P + (a.auto_shared ? a.T : 0), E_ext = a.E + (a.shared ? 1 : 0);
+    if (P_ext > kThinPairs * E_ext) return 0;
+    return a.T <= 16 ? 16 : a.T <= 32 ? 32 : 64;
+}
+
+// What launch_prefill cannot do without, and what it takes when it may choose.
+size_t prefill_workspace_min(const FwdArgs& a) { return carve(a, tile_rows(a.quant_mode), nullptr).bytes; }
+
+size_t prefill_workspace_bytes(const FwdArgs& a) {
+    const size_t m = prefill_workspace_min(a);
+    const int tr = thin_rows(a);
+    const size_t t = tr ? carve(a, tr, nullptr).bytes : 0;
+    return t > m ? t : m;
+}
 
 hipError_t launch_sort_pairs(const int32_t* pexp, int P, int E, int E_ext, int T_sh, int BM,
                              int32_t* order, int32_t* offsets, int32_t* tile_start, hipStream_t s) {
@@ -1198,7 +1117,13 @@ hipError_t launch_combine(const uint16_t* y_routed, const uint16_t* y_shared, co
 }
 
 hipError_t launch_prefill(const FwdArgs& a, void* ws, size_t ws_bytes, int phases, hipStream_t s) {
-    PfWs w = carve(a, ws);
+    // (the lower tiles' longer list must fit a fixed scratch too; else the taller ones serve)
+    int tile = thin_rows(a);
+    PfWs w = carve(a, tile ? tile : tile_rows(a.quant_mode), ws);
+    if (tile && w.bytes > ws_bytes) {
+        tile = 0;
+        w = carve(a, tile_rows(a.quant_mode), ws);
+    }
     if (w.bytes > ws_bytes) return hipErrorInvalidValue;
     const int P = a.P;
     const int T_sh = a.auto_shared ? a.T : 0;
@@ -1210,13 +1135,16 @@ hipError_t launch_prefill(const FwdArgs& a, void* ws, size_t ws_bytes, int phase
     uint16_t* y_routed = a.yun ? a.yun : w.y_routed;
     hipError_t err = hipSuccess;
     if (phases & 1) {
-        err = launch_bucket(a.pexp, P, a.E, E_ext, T_sh, tile_rows(a.quant_mode), a.g2s, a.capacity, a.host != nullptr, a.err, w.order, w.offsets,
+        err = launch_bucket(a.pexp, P, a.E, E_ext, T_sh, tile ? tile : tile_rows(a.quant_mode), a.g2s, a.capacity, a.host != nullptr, a.err, w.order, w.offsets,
                             w.tile_start, w.tinfo, s);
         if (err != hipSuccess) return err;
     }
 #define BRX_GEMM(M) (a.scale_f16 ? launch_gemm<M, true>(a, w, E_ext, Imax, y_routed, phases, s) \
                                  : launch_gemm<M, false>(a, w, E_ext, Imax, y_routed, phases, s))
-    switch (a.quant_mode) {
+    if (tile) {
+        err = launch_thin(a, ThinArgs{w.order, w.tile_start, w.tinfo, w.hbuf, y_routed, w.y_shared, E_ext, Imax,
+                                      w.mt_pad, tile}, phases, s);
+    } else switch (a.quant_mode) {
         case kModeAffine4: err = BRX_GEMM(kModeAffine4); break;
         case kModeAffine3: err = BRX_GEMM(kModeAffine3); break;
         case kModeAffine2: err = BRX_GEMM(kModeAffine2); break;
