@@ -16,160 +16,199 @@ namespace brx {
 namespace {
 
 constexpr int kRouterThreads = 256;
-constexpr int kSmallT = 64;  // up to this many tokens: one wave per (row, 4 tokens); above: token tiles
-constexpr size_t kMaxBlockLds = 160 * 1024;   // LDS one gfx950 block may allocate
+constexpr int kSmallT = 64;  // up to this many tokens: one wave per (row, 4 tokens) (5 us at 64); above: MFMA tiles (9 us)
 
 // ---------------------------------------------------------------- many tokens
-// k_router_tiled: a block takes a tile of TT tokens (staged in LDS as bf16) and a group of
-// rows; each row's weights are loaded once per block and used for all TT tokens, and a wave
-// works on two rows at once so each token's activations are converted once for both. Per
-// token the lane partials follow the same fmaf chain as k_router_logits; the TT partials are
-// reduced by a transposed butterfly that forms exactly the sums of the xor butterfly
-// (strides 32, 16, ..., 1; fp32 addition is commutative, so a[i] + a[i^s] is the same value on
-// both lanes): at stride 32 a lane keeps half of the tokens and sends the other half, at 16 a
-// quarter, and so on, so 16 tokens take 17 exchanges instead of 96. Token tau ends on lanes
-// 4 tau .. 4 tau + 3.
-template <bool WF32, int TT>
-__global__ __launch_bounds__(kRouterThreads) void k_router_tiled(
-    const uint16_t* __restrict__ x, const void* __restrict__ w, const float* __restrict__ bias,
-    const uint16_t* __restrict__ sgw, int T, int H, int E, int rows_per_block, float* __restrict__ logits) {
-    static_assert(TT == 16, "the exchange pattern below is written for 16 tokens");
-    constexpr int kNJ = 6;                      // chunks per lane per pass (one pass: H <= 3072)
-    constexpr int RW = WF32 ? 2 : 4;            // rows a wave works on at once (sharing x)
-    extern __shared__ uint4 xs4[];              // [TT][H / 8] chunks of 8 bf16
-    const int tid = threadIdx.x, lane = tid & 63, wv = tid >> 6;
-    const int t0 = blockIdx.x * TT;
-    const int nt = min(TT, T - t0);
-    const int nch = H / 8;
-    const uint4* x4 = reinterpret_cast<const uint4*>(x);
-    // kSt chunks a thread in flight at once (token rows clamped into the tile, so every load is
-    // unconditional), then the stores: a load and its store per iteration would make each of the
-    // TT * nch / kRouterThreads chunks a round trip of its own
-    {
-        constexpr int kSt = 16;
-        const int nall = TT * nch;
-        for (int i0 = 0; i0 < nall; i0 += kSt * kRouterThreads) {
-            uint4 v[kSt];
+// k_router_mfma: a block computes the logits of 16 M tokens x 16 M experts on fp32 MFMAs, in the
+// order above. v_mfma_f32_16x16x1_4b_f32 is one fused multiply-add per output and block (measured
+// bit for bit equal to fmaf chains, subnormals included), so a lane chain l is 8 of them a chunk;
+// the instruction's four blocks are the chains l, l + 16, l + 32 and l + 48 (lane group g of 16
+// lanes feeds chain l0 + 16 g). The butterfly is then: (block 0 + block 2) + (block 1 + block 3)
+// for offsets 32 and 16, and with l0 = 8 s + i (s < 2, i < 8): s for offset 8, in the wave i, and
+// the waves i ^ 4, i ^ 2 and i ^ 1 through LDS for offsets 4, 2 and 1.
+//
+// Step (s, j) copies chunks 64 j + 8 (s + 2 g) + i of the block's token rows and weight rows, four
+// runs of 128 bytes a row (256 of an fp32 row), into one slot of a ring (buffer_load ... lds; chunks
+// past the row's end and rows past the last come as zeros, which leave a chain as it is).
+//
+// Bound: the fp32 MFMA rate, 64 FMA a clock and SIMD (8 us for 2048 tokens x 128 experts x 2048),
+// and for few tiles the copies' latency. 16 x 16 tiles (M 1, two blocks a CU) while they are one
+// round of the chip; above it their copies bound them (a 16 x 16 tile reads 128 KB for 0.5 M FMA:
+// 25 us for 2048 tokens) and 32 x 32 tiles halve the bytes. The kernel this replaces formed the
+// same chains with VALU fmaf at a quarter of the MFMA's rate, converting every activation. Before
+// and after, 2048 x 128 experts: 128 tokens 13.1 -> 9.1 us, 512 15.1 -> 10.0, 2048 30.1 -> 21.9, 4096
+// 61.6 -> 44.5; 301 tokens x 257 rows 25.3 -> 12.2; 512 tokens at 2880 x 128 19.9 -> 14.1.
+typedef __attribute__((address_space(3))) void* RT_LDS;
+constexpr int kRtThreads = 512;
+template <bool WF32, int M>
+constexpr int kRtStep = 16 * M * 512 * (WF32 ? 3 : 2);   // bytes: 32 chunks of each row
+template <bool WF32>
+constexpr int kRtRing = WF32 ? 3 : 4;                     // steps in the ring
+
+template <int N>
+__device__ __forceinline__ void rt_wait_barrier() {
+    __builtin_amdgcn_s_waitcnt((N & 0xF) | (0x7 << 4) | ((N >> 4) << 14));   // vmcnt(N) lgkmcnt(0)
+    asm volatile("s_barrier" ::: "memory");
+}
+
+template <bool WF32, int M>
+__global__ __launch_bounds__(kRtThreads) void k_router_mfma(
+    const uint16_t* __restrict__ x, const void* __restrict__ w, const float* __restrict__ bias, int T, int H,
+    int E, int net, float* __restrict__ logits) {
+    constexpr int NR = kRtRing<WF32>;
+    constexpr int RT = 16 * M;
+    constexpr int XB = RT * 512;                   // x bytes of a step
+    constexpr int STEP = kRtStep<WF32, M>;
+    constexpr int NX = M, NW = WF32 ? 2 * M : M;   // 1 KB copies of a wave and step: x, weights
+    constexpr int NV = NX + NW;
+    __shared__ __attribute__((aligned(16))) uint8_t ring[NR * STEP];
+    const int tid = threadIdx.x, lane = tid & 63;
+    const int wv = __builtin_amdgcn_readfirstlane(tid >> 6);
+    // an XCD takes every expert tile of a token tile, so the x rows are read into one L2
+    const int loc = blockIdx.x / 8;
+    const int t0 = ((loc / net) * 8 + blockIdx.x % 8) * RT, e0 = (loc % net) * RT;
+    if (t0 >= T) return;
+    const int J = (H + 511) / 512, nsteps = 2 * J;
+    const uint32_t xb = (uint32_t)min(T - t0, RT) * H * 2, wb = (uint32_t)min(E - e0, RT) * H * (WF32 ? 4 : 2);
+    const uint8_t* xp = reinterpret_cast<const uint8_t*>(x) + (int64_t)t0 * H * 2;
+    const uint8_t* wp = reinterpret_cast<const uint8_t*>(w) + (int64_t)e0 * H * (WF32 ? 4 : 2);
+    const __amdgpu_buffer_rsrc_t rx =
+        __builtin_amdgcn_make_buffer_rsrc(const_cast<uint8_t*>(xp), (short)0, (int)xb, 0x00020000);
+    const __amdgpu_buffer_rsrc_t rw =
+        __builtin_amdgcn_make_buffer_rsrc(const_cast<uint8_t*>(wp), (short)0, (int)wb, 0x00020000);
+    // 16-byte slot q of a tile whose rows hold `per` slots a lane group g and chunk (1: bf16, 2:
+    // fp32 halves): slot (row r, g', i', half) holds chunk i = i' ^ (r & 7) of group g = g' ^ (r >> 3 &
+    // 1), so the 16 rows a read touches fall in distinct banks
+    auto slot_of = [&](int q, int per, int& r, int& g, int& i, int& half) __attribute__((always_inline)) {
+        half = q % per;
+        const int c = q / per;
+        r = c >> 5;
+        g = ((c >> 3) & 3) ^ ((r >> 3) & 1);
+        i = (c & 7) ^ (r & 7);
+    };
+    // issue the copies of step n = s J + j (a step past the last is all zeros and reads nothing)
+    auto issue = [&](int n) __attribute__((always_inline)) {
+        uint8_t* st = ring + (n % NR) * STEP;
+        const int s = n >= J ? 1 : 0, j = n - s * J;
+        const int lim = n < nsteps ? H / 8 : 0;
 #pragma unroll
-            for (int b = 0; b < kSt; ++b) {
-                const int i = min(i0 + b * kRouterThreads + tid, nall - 1);
-                const int t = i / nch, c = i - t * nch;
-                v[b] = x4[(int64_t)(t0 + min(t, nt - 1)) * nch + c];
-            }
+        for (int u = 0; u < NX; ++u) {
+            int r, g, i, h;
+            slot_of((wv * NX + u) * 64 + lane, 1, r, g, i, h);
+            const int c = 64 * j + 8 * (s + 2 * g) + i;
+            const uint32_t vo = c < lim ? (uint32_t)(r * H * 2 + c * 16) : xb;
+            __builtin_amdgcn_raw_ptr_buffer_load_lds(rx, (RT_LDS)(st + (wv * NX + u) * 1024), 16, vo, 0, 0, 0);
+        }
 #pragma unroll
-            for (int b = 0; b < kSt; ++b) {
-                const int i = i0 + b * kRouterThreads + tid;
-                if (i < nall) xs4[i] = i / nch < nt ? v[b] : make_uint4(0, 0, 0, 0);
+        for (int u = 0; u < NW; ++u) {
+            int r, g, i, h;
+            slot_of((wv * NW + u) * 64 + lane, WF32 ? 2 : 1, r, g, i, h);
+            const int c = 64 * j + 8 * (s + 2 * g) + i;
+            const uint32_t vo = c < lim ? (uint32_t)(WF32 ? r * H * 4 + c * 32 + h * 16 : r * H * 2 + c * 16) : wb;
+            __builtin_amdgcn_raw_ptr_buffer_load_lds(rw, (RT_LDS)(st + XB + (wv * NW + u) * 1024), 16, vo, 0, 0, 0);
+        }
+        asm volatile("" ::: "memory");
+    };
+#pragma unroll
+    for (int n = 0; n < NR - 1; ++n) issue(n);
+    const int r = lane & 15, g = lane >> 4;
+    const int q0 = r * 32 + (g ^ ((r >> 3) & 1)) * 8 + (wv ^ (r & 7));   // this wave's chunk of row r
+    auto unpack = [&](uint4 v, float (&f)[8]) __attribute__((always_inline)) {
+        const uint32_t q[4] = {v.x, v.y, v.z, v.w};
+#pragma unroll
+        for (int b = 0; b < 4; ++b) {
+            f[2 * b] = bf2f(q[b] & 0xFFFFu);
+            f[2 * b + 1] = __uint_as_float(q[b] & 0xFFFF0000u);
+        }
+    };
+    f32x16_t acc[M][M];
+    f32x4_t first[M][M];
+#pragma unroll
+    for (int m = 0; m < M; ++m)
+#pragma unroll
+        for (int n = 0; n < M; ++n) {
+#pragma unroll
+            for (int b = 0; b < 16; ++b) acc[m][n][b] = 0.0f;
+#pragma unroll
+            for (int b = 0; b < 4; ++b) first[m][n][b] = 0.0f;
+        }
+    // a block's chains of one s, complete: offsets 32 and 16
+    auto blocks_sum = [&](const f32x16_t& a, int b) __attribute__((always_inline)) {
+        return (a[b] + a[8 + b]) + (a[4 + b] + a[12 + b]);
+    };
+    for (int n = 0, slot = 0; n < nsteps; ++n) {
+        // step n landed in every wave, and step n - 1's slot is free for step n + NR - 1
+        rt_wait_barrier<(NR - 2) * NV>();
+        issue(n + NR - 1);
+        const uint8_t* st = ring + slot * STEP;
+        slot = slot + 1 == NR ? 0 : slot + 1;
+        float xf[M][8], wf[M][8];
+#pragma unroll
+        for (int m = 0; m < M; ++m) {
+            unpack(*reinterpret_cast<const uint4*>(st + (q0 + m * 512) * 16), xf[m]);
+            if constexpr (WF32) {
+                const uint8_t* p = st + XB + (q0 + m * 512) * 32;
+                const f32x4_t v0 = *reinterpret_cast<const f32x4_t*>(p), v1 = *reinterpret_cast<const f32x4_t*>(p + 16);
+#pragma unroll
+                for (int b = 0; b < 4; ++b) {
+                    wf[m][b] = v0[b];
+                    wf[m][4 + b] = v1[b];
+                }
+            } else {
+                unpack(*reinterpret_cast<const uint4*>(st + XB + (q0 + m * 512) * 16), wf[m]);
             }
         }
+#pragma unroll
+        for (int b = 0; b < 8; ++b)
+#pragma unroll
+            for (int m = 0; m < M; ++m)
+#pragma unroll
+                for (int v = 0; v < M; ++v)
+                    acc[m][v] = __builtin_amdgcn_mfma_f32_16x16x1f32(xf[m][b], wf[v][b], acc[m][v], 0, 0, 0);
+        if (n == J - 1) {
+#pragma unroll
+            for (int m = 0; m < M; ++m)
+#pragma unroll
+                for (int v = 0; v < M; ++v) {
+#pragma unroll
+                    for (int b = 0; b < 4; ++b) first[m][v][b] = blocks_sum(acc[m][v], b);
+#pragma unroll
+                    for (int b = 0; b < 16; ++b) acc[m][v][b] = 0.0f;
+                }
+        }
     }
+    // offset 8 in the wave, 4, 2 and 1 across the waves
+    rt_wait_barrier<0>();
+    float* red = reinterpret_cast<float*>(ring);
+#pragma unroll
+    for (int m = 0; m < M; ++m)
+#pragma unroll
+        for (int v = 0; v < M; ++v)
+#pragma unroll
+            for (int b = 0; b < 4; ++b)
+                red[wv * RT * RT + (16 * m + 4 * g + b) * RT + 16 * v + r] = first[m][v][b] + blocks_sum(acc[m][v], b);
     __syncthreads();
-    const int rows = E + (sgw ? 1 : 0);
-    const int r_end = min(rows, (int)(blockIdx.y + 1) * rows_per_block);
-    constexpr int kWaves = kRouterThreads / kWave;
-    for (int r0 = blockIdx.y * rows_per_block + wv * RW; r0 < r_end; r0 += kWaves * RW) {
-        // the wave's rows r0, r0 + 1 (a row past the block's range repeats the last one and is
-        // not stored)
-        float acc[RW][TT];
-#pragma unroll
-        for (int rr = 0; rr < RW; ++rr)
-#pragma unroll
-            for (int t = 0; t < TT; ++t) acc[rr][t] = 0.0f;
-        bool wf32[RW];
-#pragma unroll
-        for (int rr = 0; rr < RW; ++rr) wf32[rr] = WF32 && min(r0 + rr, r_end - 1) < E;
-        // passes of kNJ chunks per lane continue each lane's chain in chunk order
-        for (int jb = 0; jb < nch; jb += kWave * kNJ) {
-            uint4 wv4[RW][kNJ][2];
-#pragma unroll
-            for (int rr = 0; rr < RW; ++rr) {
-                const int r = min(r0 + rr, r_end - 1);
-#pragma unroll
-                for (int j = 0; j < kNJ; ++j) {
-                    const int c = min(jb + lane + kWave * j, nch - 1);
-                    if (wf32[rr]) {
-                        const uint4* p = reinterpret_cast<const uint4*>(reinterpret_cast<const float*>(w) + (int64_t)r * H + 8 * c);
-                        wv4[rr][j][0] = p[0];
-                        wv4[rr][j][1] = p[1];
-                    } else {
-                        const uint16_t* src = r < E ? reinterpret_cast<const uint16_t*>(w) + (int64_t)r * H : sgw;
-                        wv4[rr][j][0] = *reinterpret_cast<const uint4*>(src + 8 * c);
-                        wv4[rr][j][1] = make_uint4(0, 0, 0, 0);
-                    }
-                }
-            }
-#pragma unroll
-            for (int j = 0; j < kNJ; ++j) {
-                const int c = jb + lane + kWave * j;
-                if (c >= nch) continue;
-                float wf[RW][8];
-#pragma unroll
-                for (int rr = 0; rr < RW; ++rr) {
-                    if (wf32[rr]) {
-                        wf[rr][0] = __uint_as_float(wv4[rr][j][0].x); wf[rr][1] = __uint_as_float(wv4[rr][j][0].y);
-                        wf[rr][2] = __uint_as_float(wv4[rr][j][0].z); wf[rr][3] = __uint_as_float(wv4[rr][j][0].w);
-                        wf[rr][4] = __uint_as_float(wv4[rr][j][1].x); wf[rr][5] = __uint_as_float(wv4[rr][j][1].y);
-                        wf[rr][6] = __uint_as_float(wv4[rr][j][1].z); wf[rr][7] = __uint_as_float(wv4[rr][j][1].w);
-                    } else {
-                        const uint32_t ww[4] = {wv4[rr][j][0].x, wv4[rr][j][0].y, wv4[rr][j][0].z, wv4[rr][j][0].w};
-#pragma unroll
-                        for (int i = 0; i < 4; ++i) {
-                            wf[rr][2 * i] = bf2f(ww[i] & 0xFFFFu);
-                            wf[rr][2 * i + 1] = bf2f(ww[i] >> 16);
-                        }
-                    }
-                }
-                // one conversion of the token's 8 activations serves every row of the wave
-#pragma unroll
-                for (int t = 0; t < TT; ++t) {
-                    const uint4 xv = xs4[t * nch + c];
-                    const uint32_t xw[4] = {xv.x, xv.y, xv.z, xv.w};
-                    float xf[8];
-#pragma unroll
-                    for (int i = 0; i < 4; ++i) {
-                        xf[2 * i] = bf2f(xw[i] & 0xFFFFu);
-                        xf[2 * i + 1] = bf2f(xw[i] >> 16);
-                    }
-#pragma unroll
-                    for (int rr = 0; rr < RW; ++rr)
-#pragma unroll
-                        for (int i = 0; i < 8; ++i) acc[rr][t] = fmaf(xf[i], wf[rr][i], acc[rr][t]);
-                }
-            }
-        }
-#pragma unroll
-        for (int rr = 0; rr < RW; ++rr) {
-            const int r = r0 + rr;
-            // transposed butterfly: strides 32, 16, 8, 4 halve the tokens a lane keeps
-            const bool b5 = lane & 32, b4 = lane & 16, b3 = lane & 8, b2 = lane & 4;
-            float v8[8], v4[4], v2[2];
-#pragma unroll
-            for (int i = 0; i < 8; ++i) {
-                const float mine = b5 ? acc[rr][8 + i] : acc[rr][i], other = b5 ? acc[rr][i] : acc[rr][8 + i];
-                v8[i] = mine + __shfl_xor(other, 32, kWave);
-            }
-#pragma unroll
-            for (int i = 0; i < 4; ++i) {
-                const float mine = b4 ? v8[4 + i] : v8[i], other = b4 ? v8[i] : v8[4 + i];
-                v4[i] = mine + __shfl_xor(other, 16, kWave);
-            }
-#pragma unroll
-            for (int i = 0; i < 2; ++i) {
-                const float mine = b3 ? v4[2 + i] : v4[i], other = b3 ? v4[i] : v4[2 + i];
-                v2[i] = mine + __shfl_xor(other, 8, kWave);
-            }
-            float v1;
-            {
-                const float mine = b2 ? v2[1] : v2[0], other = b2 ? v2[0] : v2[1];
-                v1 = mine + __shfl_xor(other, 4, kWave);
-            }
-            v1 += __shfl_xor(v1, 2, kWave);
-            v1 += __shfl_xor(v1, 1, kWave);
-            const int tau = lane >> 2;
-            if ((lane & 3) == 0 && tau < nt && r < r_end)
-                logits[(int64_t)(t0 + tau) * (E + 1) + r] = (r < E && bias) ? v1 + bias[r] : v1;
-        }
+    for (int o = tid; o < RT * RT; o += kRtThreads) {
+        const float* p = red + o;
+        constexpr int S = RT * RT;
+        const float v = ((p[0] + p[4 * S]) + (p[2 * S] + p[6 * S])) + ((p[S] + p[5 * S]) + (p[3 * S] + p[7 * S]));
+        const int t = t0 + o / RT, e = e0 + o % RT;
+        if (t < T && e < E) logits[(int64_t)t * (E + 1) + e] = bias ? v + bias[e] : v;
     }
+}
+
+template <int M>
+hipError_t mfma_launch(const brx_layer_desc& d, const void* x, const void* w_router, const float* bias, int T,
+                       float* logits, hipStream_t s) {
+    const int net = (d.n_experts + 16 * M - 1) / (16 * M), ntt = (T + 16 * M - 1) / (16 * M);
+    dim3 grid((ntt + 7) / 8 * 8 * net), block(kRtThreads);
+    if (d.router_dtype == BRX_DT_F32)
+        hipLaunchKernelGGL((k_router_mfma<true, M>), grid, block, 0, s, (const uint16_t*)x, w_router, bias, T,
+                           d.hidden, d.n_experts, net, logits);
+    else
+        hipLaunchKernelGGL((k_router_mfma<false, M>), grid, block, 0, s, (const uint16_t*)x, w_router, bias, T,
+                           d.hidden, d.n_experts, net, logits);
+    return hipGetLastError();
 }
 
 // ---------------------------------------------------------------- small T
@@ -256,8 +295,9 @@ __global__ __launch_bounds__(WPB * kWave) void k_router_logits(
 // Top-k of one token's logits row `l` ([E + 1], the last entry the shared-gate logit) and its
 // routing weights, by the calling wave.
 template <int kPer>
-__device__ __forceinline__ void topk_row(const float* __restrict__ l, int t, int E, int k, const RouteRule& rr,
-                                         int has_sg, int32_t* __restrict__ out_idx,
+__device__ __forceinline__ void topk_row(const float* __restrict__ l, const uint16_t* __restrict__ x,
+                                         const uint16_t* __restrict__ sgw, int t, int H, int E, int k,
+                                         const RouteRule& rr, int has_sg, int32_t* __restrict__ out_idx,
                                          float* __restrict__ out_w, float* __restrict__ out_sg) {
     const int lane = threadIdx.x & 63;
     float v[kPer];
@@ -265,6 +305,32 @@ __device__ __forceinline__ void topk_row(const float* __restrict__ l, int t, int
     for (int i = 0; i < kPer; ++i) {
         const int e = lane + kWave * i;
         v[i] = e < E ? l[e] : 0.0f;
+    }
+    // the shared gate's logit, where the logits come without it: the wave's lanes are its chains
+    float gate = 0.0f;
+    if (sgw) {
+        constexpr int kG = 4;                       // chunks a lane has in flight
+        for (int c0 = lane; c0 < H / 8; c0 += kWave * kG) {
+            uint4 xv[kG], gv[kG];
+#pragma unroll
+            for (int u = 0; u < kG; ++u) {
+                const int c = min(c0 + kWave * u, H / 8 - 1);
+                xv[u] = *reinterpret_cast<const uint4*>(x + (int64_t)t * H + 8 * c);
+                gv[u] = *reinterpret_cast<const uint4*>(sgw + 8 * c);
+            }
+#pragma unroll
+            for (int u = 0; u < kG; ++u) {
+                if (c0 + kWave * u >= H / 8) break;
+                const uint32_t xw[4] = {xv[u].x, xv[u].y, xv[u].z, xv[u].w};
+                const uint32_t gw[4] = {gv[u].x, gv[u].y, gv[u].z, gv[u].w};
+#pragma unroll
+                for (int i = 0; i < 4; ++i) {
+                    gate = fmaf(bf2f(xw[i] & 0xFFFFu), bf2f(gw[i] & 0xFFFFu), gate);
+                    gate = fmaf(bf2f(xw[i] >> 16), bf2f(gw[i] >> 16), gate);
+                }
+            }
+        }
+        gate = wave_sum_xor(gate);
     }
     int my_id;
     float my_v;
@@ -274,17 +340,18 @@ __device__ __forceinline__ void topk_row(const float* __restrict__ l, int t, int
         out_idx[(int64_t)t * k + lane] = my_id;
         out_w[(int64_t)t * k + lane] = wt;
     }
-    if (lane == 0 && has_sg && out_sg) out_sg[t] = 1.0f / (1.0f + expf(-l[E]));
+    if (lane == 0 && has_sg && out_sg) out_sg[t] = 1.0f / (1.0f + expf(-(sgw ? gate : l[E])));
 }
 
-// One wave per token over logits [T][E + 1].
+// One wave per token over logits [T][E + 1]; with `sgw` given it also forms the shared gate's logit.
 template <int kPer>
 __global__ __launch_bounds__(kRouterThreads) void k_router_topk(
-    const float* __restrict__ logits, int T, int E, int k, RouteRule rr, int has_sg,
-    int32_t* __restrict__ out_idx, float* __restrict__ out_w, float* __restrict__ out_sg) {
+    const float* __restrict__ logits, const uint16_t* __restrict__ x, const uint16_t* __restrict__ sgw, int T, int H,
+    int E, int k, RouteRule rr, int has_sg, int32_t* __restrict__ out_idx, float* __restrict__ out_w,
+    float* __restrict__ out_sg) {
     const int t = blockIdx.x * (kRouterThreads / kWave) + (threadIdx.x >> 6);
     if (t >= T) return;
-    topk_row<kPer>(logits + (int64_t)t * (E + 1), t, E, k, rr, has_sg, out_idx, out_w, out_sg);
+    topk_row<kPer>(logits + (int64_t)t * (E + 1), x, sgw, t, H, E, k, rr, has_sg, out_idx, out_w, out_sg);
 }
 
 template <bool WF32>
@@ -299,13 +366,13 @@ hipError_t logits_launch(const brx_layer_desc& d, const void* x, const void* w_r
     return hipGetLastError();
 }
 
-hipError_t topk_launch(const brx_layer_desc& d, int T, int has_sg, const float* logits, const float* bias,
-                       int32_t* out_idx, float* out_w, float* out_sg, hipStream_t s) {
+hipError_t topk_launch(const brx_layer_desc& d, int T, int has_sg, const float* logits, const void* x,
+                       const void* sgw, const float* bias, int32_t* out_idx, float* out_w, float* out_sg, hipStream_t s) {
     const int E = d.n_experts;
     const RouteRule rr = route_rule(d, bias);
     dim3 grid((T + 3) / 4), block(kRouterThreads);
-#define BRX_TOPK(KP) hipLaunchKernelGGL(k_router_topk<KP>, grid, block, 0, s, logits, T, E, d.top_k, \
-                                        rr, has_sg, out_idx, out_w, out_sg)
+#define BRX_TOPK(KP) hipLaunchKernelGGL(k_router_topk<KP>, grid, block, 0, s, logits, (const uint16_t*)x, \
+                                        (const uint16_t*)sgw, T, d.hidden, E, d.top_k, rr, has_sg, out_idx, out_w, out_sg)
     if (E <= 64) BRX_TOPK(1);
     else if (E <= 128) BRX_TOPK(2);
     else if (E <= 256) BRX_TOPK(4);
@@ -333,39 +400,17 @@ hipError_t launch_router(const brx_layer_desc& d, const void* x, const void* w_r
                          const float* bias, const void* sgw, int T, int32_t* out_idx,
                          float* out_w, float* out_sg, float* ws_logits, hipStream_t s) {
     if (T <= 0) return hipSuccess;
-    const bool f32 = d.router_dtype == BRX_DT_F32;
-    // the tiled kernel stages 16 token rows of x in LDS, 32 * H bytes: within a block's 160 KB up
-    // to H = 5120. Wider layers route every token tile with the small-T kernel (the same per-lane
-    // chains and butterfly, so the same bits).
-    if (T <= kSmallT || (size_t)32 * d.hidden > kMaxBlockLds) {
+    if (T <= kSmallT) {
         hipError_t e = launch_router_logits(d, x, w_router, bias, sgw, T, ws_logits, s);
         if (e != hipSuccess) return e;
-        return topk_launch(d, T, sgw ? 1 : 0, ws_logits, bias, out_idx, out_w, out_sg, s);
+        return topk_launch(d, T, sgw ? 1 : 0, ws_logits, nullptr, nullptr, bias, out_idx, out_w, out_sg, s);
     }
-    // many tokens: logits by token tiles, then the same top-k kernel
-    // rows per block: 32 (each weight row read once per 16-token tile, by one wave), fewer
-    // when there are too few token tiles for one round of blocks over the 256 CUs (a wave then
-    // takes fewer rows; every block stages its token tile, so a second round would stage it
-    // again for no more work in flight). Blocks per CU: as many staged tiles as fit in a CU's
-    // 160 KB (two at H 2048, one at H 2880)
-    constexpr int TT = 16;
-    const int rows = d.n_experts + (sgw ? 1 : 0);
-    const int tiles = (T + TT - 1) / TT;
-    const size_t lds = sizeof(uint16_t) * (size_t)TT * d.hidden;
-    const int per_cu = (int)(kMaxBlockLds / lds) < 2 ? 1 : 2;
-    int RPB = 32;
-    while (RPB > 4 && tiles * ((rows + RPB - 1) / RPB) < 256 * per_cu) RPB /= 2;
-    dim3 grid(tiles, (rows + RPB - 1) / RPB);
     const float* lbias = d.route_mode >= BRX_ROUTE_SIGMOID_TOPK ? nullptr : bias;
-    if (f32)
-        hipLaunchKernelGGL((k_router_tiled<true, TT>), grid, dim3(kRouterThreads), lds, s, (const uint16_t*)x,
-                           w_router, lbias, (const uint16_t*)sgw, T, d.hidden, d.n_experts, RPB, ws_logits);
-    else
-        hipLaunchKernelGGL((k_router_tiled<false, TT>), grid, dim3(kRouterThreads), lds, s, (const uint16_t*)x,
-                           w_router, lbias, (const uint16_t*)sgw, T, d.hidden, d.n_experts, RPB, ws_logits);
-    hipError_t e = hipGetLastError();
+    const int64_t tiles16 = (int64_t)((T + 15) / 16) * ((d.n_experts + 15) / 16);
+    hipError_t e = tiles16 <= 512 ? mfma_launch<1>(d, x, w_router, lbias, T, ws_logits, s)
+                                  : mfma_launch<2>(d, x, w_router, lbias, T, ws_logits, s);
     if (e != hipSuccess) return e;
-    return topk_launch(d, T, sgw ? 1 : 0, ws_logits, bias, out_idx, out_w, out_sg, s);
+    return topk_launch(d, T, sgw ? 1 : 0, ws_logits, x, sgw, bias, out_idx, out_w, out_sg, s);
 }
 
 }  // namespace brx
