@@ -476,9 +476,8 @@ __device__ __forceinline__ float sigmoid_f(float v) { return 1.0f / (1.0f + exp_
 // the logit itself (softmax modes) or sigmoid(logit) + bias (sigmoid modes); with groups
 // (n_group > 1) the experts outside the topk_group best groups are then taken out (softmax:
 // -inf; sigmoid: 0). A group's score is its largest logit (softmax) or the sum of its two
-// largest selection values (sigmoid; the second largest is the largest of the others after one
-// holder of the maximum, the lowest id, is set aside); groups rank by score, ties to the lower
-// group, as the top-k does.
+// largest selection values (sigmoid); groups rank by score, ties to the lower group, as the
+// top-k does.
 template <int kPer>
 __device__ __forceinline__ void route_values(const float v[kPer], const RouteRule& rr, int E, float c[kPer]) {
     const int lane = threadIdx.x & (kWave - 1);
@@ -495,34 +494,38 @@ __device__ __forceinline__ void route_values(const float v[kPer], const RouteRul
 #pragma unroll
     for (int i = 0; i < kPer; ++i) c[i] = sig ? sigmoid_f(v[i]) + bv[i] : v[i];
     if (rr.n_group <= 1) return;
+    // all groups at once: LP lanes a group gather its values (the lane and register that hold an
+    // expert are e % 64 and e / 64) and merge their two largest; NaN counts as -inf. (One group
+    // after the other, each two wave reductions, the 8-group ranking of 301 tokens took 13.4 us against 10.4.)
     const int G = E / rr.n_group;
-    float gs = -__builtin_inff();          // lane g: group g's score
-    for (int g = 0; g < rr.n_group; ++g) {
-        float lm = -__builtin_inff();
-        bool mem[kPer];
+    int lg = 0;
+    while ((1 << lg) < rr.n_group) ++lg;
+    const int LP = kWave >> lg, grp = lane >> (6 - lg), s = lane & (LP - 1);
+    float m1 = -__builtin_inff(), m2 = -__builtin_inff();
+    for (int q = s; q < G + s; q += LP) {       // (uniform trip count up to one past-the-end step)
+        const int e = min(grp * G + q, E - 1);
+        float t = -__builtin_inff();
 #pragma unroll
         for (int i = 0; i < kPer; ++i) {
-            const int e = lane + kWave * i;
-            mem[i] = e >= g * G && e < (g + 1) * G;
-            if (mem[i]) lm = fmaxf(lm, c[i]);
+            const float v = __shfl(c[i], e & (kWave - 1), kWave);
+            if ((e >> 6) == i) t = v;
         }
-        const float m1 = wave_max(lm);
-        float score = m1;
-        if (sig) {
-            int first = -1;
-#pragma unroll
-            for (int i = 0; i < kPer; ++i) {
-                const uint64_t b = __ballot(mem[i] && c[i] == m1);
-                if (first < 0 && b) first = kWave * i + __builtin_ctzll(b);
-            }
-            float l2 = -__builtin_inff();
-#pragma unroll
-            for (int i = 0; i < kPer; ++i)
-                if (mem[i] && lane + kWave * i != first) l2 = fmaxf(l2, c[i]);
-            score = m1 + wave_max(l2);
-        }
-        if (lane == g) gs = score;
+        if (q >= G || grp >= rr.n_group || t != t) t = -__builtin_inff();
+        m2 = fmaxf(m2, fminf(m1, t));
+        m1 = fmaxf(m1, t);
     }
+    auto merge = [&](float o1, float o2) __attribute__((always_inline)) {
+        m2 = fmaxf(fminf(m1, o1), fmaxf(m2, o2));
+        m1 = fmaxf(m1, o1);
+    };
+    if (LP >= 2) merge(dpp_f<0xB1>(m1), dpp_f<0xB1>(m2));
+    if (LP >= 4) merge(dpp_f<0x4E>(m1), dpp_f<0x4E>(m2));
+    if (LP >= 8) merge(dpp_f<0x141>(m1), dpp_f<0x141>(m2));
+    if (LP >= 16) merge(dpp_f<0x140>(m1), dpp_f<0x140>(m2));
+    if (LP >= 32) merge(lane_xor16_f(m1), lane_xor16_f(m2));
+    const float score = sig ? m1 + m2 : m1;
+    float gs = __shfl(score, min(lane, rr.n_group - 1) << (6 - lg), kWave);   // lane g: group g's score
+    if (lane >= rr.n_group) gs = -__builtin_inff();
     uint64_t keep = 0;
     bool live = lane < rr.n_group;
     for (int r = 0; r < rr.topk_group; ++r) {

@@ -42,113 +42,116 @@ constexpr int kBK = 64;           // K step
 constexpr int kThreads = 256;
 
 // ------------------------------------------------------------------ bucketing
-// Pairs are read coalesced: in each pass of kBucketPass pairs, wave w takes the 1024 pairs
-// [w * 1024, w * 1024 + 1024) and its lane l the pairs l + 64 i (i < 16), so a load
-// instruction reads 64 consecutive pairs, and the histogram's LDS atomics of one instruction
-// (8 tokens x top-8, distinct experts within a token) hit one address at most 8 times. The
-// stable compaction of a pass is 16 ballots per wave and one scan of the 16 wave totals.
+// Pairs are read coalesced: in each pass of 1024 PER pairs, wave w takes the 64 PER pairs
+// [64 PER w, 64 PER (w + 1)) and its lane l the pairs l + 64 i (i < PER), so a load instruction
+// reads 64 consecutive pairs, and the histogram's LDS atomics of one instruction (8 tokens x
+// top-8, distinct experts within a token) hit one address at most 8 times. The stable compaction
+// of a pass is PER ballots per wave and one scan of the 16 wave totals. PER is 16 for many pairs
+// (one pass of 2048 top-8 tokens), and 2 or 4 for up to 2048 or 8192: there the launch is bound by
+// its cold code and chain of barriers, not by the pairs (one kernel of 16 pairs a lane, 10 KB of
+// code, took 7.8 us for 256 pairs and 13.5 for 2709 pairs of 257 experts; now 3.6 and 4.8).
 constexpr int kBucketThreads = 1024;
-constexpr int kBucketPer = 16;                                 // pairs per lane per pass
-constexpr int kBucketWaveRun = kWave * kBucketPer;            // pairs per wave per pass
-constexpr int kBucketPass = kBucketThreads * kBucketPer;
 constexpr int kBucketListMax = 8192;                          // pairs an LDS list may hold
 
-// The experts of a lane's pairs pb + 64 i (i < kBucketPer; id E for the shared expert's pairs
-// past the P routed ones). The loads are unconditional (index clamped into the routed pairs), so
-// a lane's sixteen are in flight together rather than one round trip each.
+// The experts of a lane's pairs pb + 64 i (i < PER; id E for the shared expert's pairs past the P
+// routed ones). The loads are unconditional (index clamped into the routed pairs), so a lane's
+// are in flight together rather than one round trip each.
+template <int PER>
 __device__ __forceinline__ void bucket_experts(const int32_t* __restrict__ pexp, int pb, int P, int E, int emax,
-                                               int ex[kBucketPer]) {
+                                               int ex[PER]) {
     if (P > 0) {   // uniform
 #pragma unroll
-        for (int i = 0; i < kBucketPer; ++i) ex[i] = pexp[min(pb + i * kWave, P - 1)];
+        for (int i = 0; i < PER; ++i) ex[i] = pexp[min(pb + i * kWave, P - 1)];
     }
 #pragma unroll
-    for (int i = 0; i < kBucketPer; ++i) ex[i] = pb + i * kWave < P ? min(max(ex[i], 0), emax) : E;
+    for (int i = 0; i < PER; ++i) ex[i] = pb + i * kWave < P ? min(max(ex[i], 0), emax) : E;
 }
 
+template <int PER>
 __global__ __launch_bounds__(kBucketThreads) void k_bucket(const int32_t* __restrict__ pexp, int P, int E,
-                                                           int E_ext, int T_sh, int BM,
+                                                           int E_ext, int T_sh, int lbm,
                                                            const int32_t* __restrict__ g2s, int capacity,
                                                            int host, int32_t* __restrict__ err,
                                                            int32_t* __restrict__ order,
                                                            int32_t* __restrict__ offsets,
                                                            int32_t* __restrict__ tile_start,
                                                            int4* __restrict__ tinfo, int lcap) {
-    // E_ext = E + 1 when a shared expert exists (id E); T_sh shared pairs follow the P routed.
-    // LDS: the histogram [E_ext], then a list of up to lcap of this expert's pairs.
+    // E_ext = E + 1 when a shared expert exists (id E); T_sh shared pairs follow the P routed; the M
+    // tile height is 1 << lbm. LDS: the histogram [E_ext], then a list of up to lcap of this
+    // expert's pairs.
     extern __shared__ int32_t hist[];
     int32_t* list = hist + E_ext;
     constexpr int kNw = kBucketThreads / kWave;
+    constexpr int kPass = kBucketThreads * PER;
     __shared__ int32_t wsum[kNw];
     __shared__ int32_t base_s[3];
+    const int BM = 1 << lbm;
     const int P_ext = P + T_sh;
     const int emax = E_ext - 1;
     const int e = blockIdx.x;
     const int tid = threadIdx.x, lane = tid & 63, wv = tid >> 6;
     const uint64_t below = (1ull << lane) - 1ull;
+    int slot = 0;   // the slot code: a slot, -2 - e for an expert read from host backing
+    if (tinfo && e < E && g2s) {
+        const int v = g2s[e];
+        slot = v >= 0 ? min(v, capacity - 1) : (host ? -2 - e : kAbsentCode);
+    }
     for (int i = tid; i < E_ext; i += kBucketThreads) hist[i] = 0;
     __syncthreads();
-    // one pass over the pairs: the histogram of every pair's expert (each block needs all counts
-    // below its own expert) and the stable (pair-order) compaction of this expert's pairs into
-    // the LDS list, pair order = (pass, wave, i, lane)
-    int run = 0;
-    for (int p0 = 0; p0 < P_ext; p0 += kBucketPass) {
-        const int pb = p0 + wv * kBucketWaveRun + lane;
-        int ex[kBucketPer];
-        bucket_experts(pexp, pb, P, E, emax, ex);
+    // This expert's pairs of the pass at p0, in pair order (pass, wave, i, lane), handed to put(place,
+    // pair) from place `run` on; returns the pass's count. COUNT also counts every pair's expert
+    // into the histogram (each block needs all counts below its own expert).
+    auto compact = [&](int p0, int run, auto count, auto put) __attribute__((always_inline)) {
+        const int pb = p0 + wv * (kWave * PER) + lane;
+        int ex[PER];
+        bucket_experts<PER>(pexp, pb, P, E, emax, ex);
+        uint64_t m[PER];
+        int cnt = 0;
 #pragma unroll
-        for (int i = 0; i < kBucketPer; ++i)
-            if (pb + i * kWave < P_ext) atomicAdd(&hist[ex[i]], 1);
-        {
-            uint64_t m[kBucketPer];
-            int cnt = 0;
-#pragma unroll
-            for (int i = 0; i < kBucketPer; ++i) {
-                m[i] = __ballot(pb + i * kWave < P_ext && ex[i] == e);
-                cnt += __popcll(m[i]);
-            }
-            if (lane == 0) wsum[wv] = cnt;
-            __syncthreads();
-            int before = 0, total = 0;
-#pragma unroll
-            for (int w = 0; w < kNw; ++w) {
-                const int v = wsum[w];
-                before += w < wv ? v : 0;
-                total += v;
-            }
-            int dst = run + before;
-#pragma unroll
-            for (int i = 0; i < kBucketPer; ++i) {
-                const int q = dst + __popcll(m[i] & below);
-                if (((m[i] >> lane) & 1ull) && q < lcap) list[q] = pb + i * kWave;
-                dst += __popcll(m[i]);
-            }
-            run += total;
-            __syncthreads();
+        for (int i = 0; i < PER; ++i) {
+            const bool in = pb + i * kWave < P_ext;
+            if (decltype(count)::value && in) atomicAdd(&hist[ex[i]], 1);
+            m[i] = __ballot(in && ex[i] == e);
+            cnt += __popcll(m[i]);
         }
-    }
-    __syncthreads();
+        if (lane == 0) wsum[wv] = cnt;
+        __syncthreads();
+        // lane w < 16: the total of wave w; its prefix below this wave and the pass's total
+        const int incl = wave_incl_scan(lane < kNw ? wsum[lane] : 0);
+        const int before = __builtin_amdgcn_readlane(incl, max(wv - 1, 0));
+        const int total = __builtin_amdgcn_readlane(incl, kNw - 1);
+        int dst = run + (wv > 0 ? before : 0);
+#pragma unroll
+        for (int i = 0; i < PER; ++i) {
+            if ((m[i] >> lane) & 1ull) put(dst + __popcll(m[i] & below), pb + i * kWave);
+            dst += __popcll(m[i]);
+        }
+        __syncthreads();
+        return total;
+    };
+    int run = 0;
+    for (int p0 = 0; p0 < P_ext; p0 += kPass)
+        run += compact(p0, run, std::true_type{}, [&](int q, int p) { if (q < lcap) list[q] = p; });
     if (wv == 0) {
         // expert e's run offset (counts of the experts before it) and its tiles' places in the
         // tile list, which holds the tiles of more than BM / 2 rows of every expert first, then
         // the smaller ones (at most one per expert, its last), each class in expert order, so
-        // the GEMMs take the long tiles first
-        int off = 0, big = 0, small = 0, big_all = 0, small_all = 0;
+        // the GEMMs take the long tiles first. The two counts of a class pair share a word (a
+        // call has fewer than 2^16 small tiles, one an expert).
+        int off = 0, below_e = 0, big_all = 0, small_all = 0, big = 0;
         for (int j = lane; j < E_ext; j += 64) {
-            const int n = hist[j], r = n % BM;
-            const int nb = n / BM + (r > BM / 2 ? 1 : 0), ns = (r > 0 && r <= BM / 2) ? 1 : 0;
-            if (j < e) { off += n; big += nb; small += ns; }
+            const int n = hist[j], r = n & (BM - 1);
+            const int nb = (n >> lbm) + (r > BM / 2 ? 1 : 0), ns = (r > 0 && r <= BM / 2) ? 1 : 0;
+            if (j < e) { off += n; big += nb; below_e += ns; }
             big_all += nb;
             small_all += ns;
         }
-        for (int sft = 32; sft >= 1; sft >>= 1) {
-            off += __shfl_xor(off, sft, 64);
-            big += __shfl_xor(big, sft, 64);
-            small += __shfl_xor(small, sft, 64);
-            big_all += __shfl_xor(big_all, sft, 64);
-            small_all += __shfl_xor(small_all, sft, 64);
-        }
-        if (lane == 0) {
+        off = wave_incl_scan(off);          // lane 63 holds the sums
+        big = wave_incl_scan(big);
+        big_all = wave_incl_scan(big_all);
+        const int small2 = wave_incl_scan(below_e | (small_all << 16));
+        if (lane == 63) {
+            const int small = small2 & 0xFFFF, smalls = small2 >> 16;
             base_s[0] = off;
             base_s[1] = big;
             base_s[2] = big_all + small;
@@ -156,7 +159,7 @@ __global__ __launch_bounds__(kBucketThreads) void k_bucket(const int32_t* __rest
             tile_start[e] = big;
             if (e == E_ext - 1) {
                 offsets[E_ext] = P_ext;
-                tile_start[E_ext] = big_all + small_all;   // tiles in all (what the GEMMs read)
+                tile_start[E_ext] = big_all + smalls;   // tiles in all (what the GEMMs read)
             }
         }
     }
@@ -164,14 +167,9 @@ __global__ __launch_bounds__(kBucketThreads) void k_bucket(const int32_t* __rest
     const int n = hist[e], off = base_s[0];
     if (tinfo) {
         const int big = base_s[1], small = base_s[2];
-        int slot = 0;
-        if (e < E && g2s) {   // the slot code: a slot, -2 - e for an expert read from host backing
-            const int v = g2s[e];
-            slot = v >= 0 ? min(v, capacity - 1) : (host ? -2 - e : kAbsentCode);
-            if (slot == kAbsentCode && n > 0 && tid == 0 && err) {
-                err[1] = e;
-                err[0] = 1;
-            }
+        if (slot == kAbsentCode && n > 0 && tid == 0 && err) {
+            err[1] = e;
+            err[0] = 1;
         }
         for (int j = tid; j * BM < n; j += kBucketThreads) {
             const int rows = min(BM, n - j * BM);
@@ -184,36 +182,10 @@ __global__ __launch_bounds__(kBucketThreads) void k_bucket(const int32_t* __rest
         return;
     }
     // the expert's pairs did not fit the LDS list: a second pass compacts straight into the run
-    run = off;
-    for (int p0 = 0; p0 < P_ext; p0 += kBucketPass) {
-        const int pb = p0 + wv * kBucketWaveRun + lane;
-        uint64_t m[kBucketPer];
-        int cnt = 0;
-        int ex[kBucketPer];
-        bucket_experts(pexp, pb, P, E, emax, ex);
-#pragma unroll
-        for (int i = 0; i < kBucketPer; ++i) {
-            const int p = pb + i * kWave;
-            m[i] = __ballot(p < P_ext && ex[i] == e);
-            cnt += __popcll(m[i]);
-        }
-        if (lane == 0) wsum[wv] = cnt;
-        __syncthreads();
-        int before = 0, total = 0;
-#pragma unroll
-        for (int w = 0; w < kNw; ++w) {
-            const int v = wsum[w];
-            before += w < wv ? v : 0;
-            total += v;
-        }
-        int dst = run + before;
-#pragma unroll
-        for (int i = 0; i < kBucketPer; ++i) {
-            if ((m[i] >> lane) & 1ull) order[dst + __popcll(m[i] & below)] = pb + i * kWave;
-            dst += __popcll(m[i]);
-        }
-        run += total;
-        __syncthreads();
+    if constexpr (PER > 4) {
+        run = off;
+        for (int p0 = 0; p0 < P_ext; p0 += kPass)
+            run += compact(p0, run, std::false_type{}, [&](int q, int p) { order[q] = p; });
     }
 }
 
@@ -1070,8 +1042,14 @@ hipError_t launch_bucket(const int32_t* pexp, int P, int E, int E_ext, int T_sh,
     // an expert with more takes a second pass over the pairs
     const int P_ext = P + T_sh;
     const int lcap = P_ext < kBucketListMax ? P_ext : kBucketListMax;
-    hipLaunchKernelGGL(k_bucket, dim3(E_ext), dim3(kBucketThreads), sizeof(int32_t) * (E_ext + lcap), s, pexp, P,
-                       E, E_ext, T_sh, BM, g2s, capacity, host, err, order, offsets, tile_start, tinfo, lcap);
+    const size_t lds = sizeof(int32_t) * (E_ext + lcap);
+    const int lbm = __builtin_ctz(BM);
+#define BRX_BUCKET(PER) hipLaunchKernelGGL(k_bucket<PER>, dim3(E_ext), dim3(kBucketThreads), lds, s, pexp, P, E, E_ext, \
+                                           T_sh, lbm, g2s, capacity, host, err, order, offsets, tile_start, tinfo, lcap)
+    if (P_ext <= 2 * kBucketThreads) BRX_BUCKET(2);
+    else if (P_ext <= kBucketListMax) BRX_BUCKET(4);    // (a list that holds every pair: no second pass)
+    else BRX_BUCKET(16);
+#undef BRX_BUCKET
     return hipGetLastError();
 }
 
