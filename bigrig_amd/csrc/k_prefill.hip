@@ -19,9 +19,11 @@
 //              bucketed order.  KIND 1 (down):
 //              A = h rows, B = down weights of 256 output columns; the epilogue stores each
 //              pair's bf16 row at its (token, k) position.  A is staged through LDS, B is
-//              dequantized from its packed codes (affine 2-8 bits, MXFP4; bf16 as loaded) into MFMA
+//              dequantized from its packed codes (affine 2-8 bits, MXFP4) into MFMA
 //              operand registers; fp32 accumulators (details at the kernel). M tiles are 128
-//              rows (64 for 6- and 8-bit codes and bf16 weights).
+//              rows (64 for 6- and 8-bit codes).
+//   k_thin_gemm (k_thin.hip) takes the calls of few pairs an expert, k_dense_gemm (k_dense.hip)
+//              those of unquantized bf16 experts.
 //   k_combine  out[t] = sum_j w[t,j] * y[t,j] (+ shared_gate[t] * y_shared[t]), k-ordered.
 // Every output element is one MFMA accumulation over K in a fixed K order, so a row's value
 // does not depend on which other pairs share its tile.
@@ -37,8 +39,6 @@
 namespace brx {
 namespace {
 
-constexpr int kBM = 128;          // pairs per M tile
-constexpr int kBK = 64;           // K step
 constexpr int kThreads = 256;
 
 // ------------------------------------------------------------------ bucketing
@@ -221,11 +221,6 @@ __global__ __launch_bounds__(kBucketThreads) void k_bucket(const int32_t* __rest
 //   (kk = 3: A(s + 1) kk 0) from LDS
 // The MFMA-interleaved VALU code is plain C++ so that the compiler's MFMA hazard checks cover
 // it.
-constexpr int kGemmWaves = 4;
-constexpr int kGemmThreads = 64 * kGemmWaves;
-constexpr int kNJ = 2;                       // 32-column fragments per wave
-constexpr int kWaveN = 32 * kNJ;             // columns per wave
-constexpr int kBlockN = kGemmWaves * kWaveN; // columns per block
 constexpr int kNS = 4;                       // LDS ring stages (even: see pf_tile)
 constexpr int kStA = kBM * kBK * 2;          // stage bytes: A tile
 constexpr int kStS = kBlockN * 4 * 2;        // scale and bias per row, one 32-bit LDS slot each
@@ -249,125 +244,11 @@ constexpr int loads_after(int ns, int nv0, int nv1, int par) {
     return n;
 }
 
-// M tile height: 128 rows, or 64 for 6- and 8-bit codes and bf16 weights, whose B words (48, 64
-// and 128 registers over the ring) leave no room for the accumulators of a 128-row tile at two
+// M tile height: 128 rows, or 64 for 6- and 8-bit codes, whose B words (48 and 64 registers over
+// the ring) leave no room for the accumulators of a 128-row tile at two
 // blocks per CU
 template <int MODE>
 constexpr int kTileRows = kBits<MODE> >= 6 ? 64 : 128;
-
-// The gate/up epilogue of one activation rule: act(gate + bias, up + bias) (or SiLU(fc1 + bias))
-// of every accumulator into the LDS tile T (row stride TS elements), NaN for an absent expert.
-// A gated tile's wave holds 32 features: fragment 0 their gate rows, fragment 1 their up rows;
-// a two-layer expert's fragment nj holds 32 fc1 features of its own. Element i of a 32 x 32
-// fragment is row 8 (i / 4) + 4 kh + i % 4, column l32.
-template <int MR, int ACT>
-__device__ __forceinline__ void pf_store_h(const FwdArgs& a, const Layout& L, const uint8_t* base, int inter,
-                                           bool absent, int nt, const f32x16_t (&acc)[MR][kNJ], uint16_t* T,
-                                           int wv, int kh, int l32) {
-    const float nan = absent_nan();
-    if constexpr (ACT == BRX_ACT_SILU_MLP) {
-        constexpr int TS = kBlockN + 8;
-#pragma unroll
-        for (int nj = 0; nj < kNJ; ++nj) {
-            const int fl = nj * 128 + wv * 32 + l32;
-            const int f = min(nt * kBlockN + fl, inter - 1);
-            const float bg = L.p[0].bias >= 0 ? bf2f(reinterpret_cast<const uint16_t*>(base + L.p[0].bias)[f]) : 0.f;
-#pragma unroll
-            for (int mi = 0; mi < MR; ++mi) {
-#pragma unroll
-                for (int i = 0; i < 16; ++i) {
-                    float h = act_fixed<ACT>(acc[mi][nj][i] + bg, 0.f, a.alpha, a.limit);
-                    h = absent ? nan : h;
-                    T[(mi * 32 + 8 * (i >> 2) + 4 * kh + (i & 3)) * TS + fl] = __builtin_bit_cast(uint16_t, (__bf16)h);
-                }
-            }
-        }
-    } else {
-        constexpr int TS = kBlockN / 2 + 8;
-        const int fl = wv * (kWaveN / 2) + l32;
-        const int f = min(nt * (kBlockN / 2) + fl, inter - 1);
-        float bg = 0.f, bu = 0.f;
-        if (L.p[0].bias >= 0) {
-            bg = bf2f(reinterpret_cast<const uint16_t*>(base + L.p[0].bias)[f]);
-            bu = bf2f(reinterpret_cast<const uint16_t*>(base + L.p[1].bias)[f]);
-        }
-#pragma unroll
-        for (int mi = 0; mi < MR; ++mi) {
-#pragma unroll
-            for (int i = 0; i < 16; ++i) {
-                float h = act_fixed<ACT>(acc[mi][0][i] + bg, acc[mi][1][i] + bu, a.alpha, a.limit);
-                h = absent ? nan : h;
-                T[(mi * 32 + 8 * (i >> 2) + 4 * kh + (i & 3)) * TS + fl] = __builtin_bit_cast(uint16_t, (__bf16)h);
-            }
-        }
-    }
-}
-
-// The epilogue of a GEMM tile: MR x kNJ fragments of fp32 accumulators per wave go through LDS
-// (`ring`, free once the caller has waited for every copy into it and synchronised) so the
-// global stores are 16-byte chunks of contiguous row segments. KIND 0: the activation (one code
-// path per rule, chosen once per tile) stored as bf16 h rows at their bucketed positions; KIND 1:
-// + bias, each pair's row stored at its (token, k) position (dst_s). An absent expert's h rows
-// are NaN.
-template <int KIND, int MR>
-__device__ __forceinline__ void pf_store(const FwdArgs& a, const Layout& L, const uint8_t* base, bool mlp, int inter,
-                                         int slot, int nt, int m0, int rows, const f32x16_t (&acc)[MR][kNJ],
-                                         uint8_t* ring, const int32_t* dst_s, uint16_t* __restrict__ hbuf,
-                                         int hstride, uint16_t* __restrict__ y_routed,
-                                         uint16_t* __restrict__ y_shared) {
-    constexpr int MF = MR * 2;
-    const int H = a.H;
-    const int tid = threadIdx.x, lane = tid & 63;
-    const int wv = __builtin_amdgcn_readfirstlane(tid >> 6);
-    const int kh = lane >> 5, l32 = lane & 31;
-    uint16_t* T = reinterpret_cast<uint16_t*>(ring);
-    if constexpr (KIND == 0) {
-        const bool absent = slot == kAbsentCode;
-        if (mlp)
-            pf_store_h<MR, BRX_ACT_SILU_MLP>(a, L, base, inter, absent, nt, acc, T, wv, kh, l32);
-        else if (a.act == BRX_ACT_SWIGLU_CLAMPED)
-            pf_store_h<MR, BRX_ACT_SWIGLU_CLAMPED>(a, L, base, inter, absent, nt, acc, T, wv, kh, l32);
-        else
-            pf_store_h<MR, BRX_ACT_SWIGLU>(a, L, base, inter, absent, nt, acc, T, wv, kh, l32);
-        lds_barrier();
-        // a two-layer expert's tile holds kBlockN features, a gated one's kBlockN / 2
-        const int fpb = mlp ? kBlockN : kBlockN / 2;
-        const int TS = fpb + 8;
-        const int CH = fpb / 8;
-        for (int c = tid; c < MF * 16 * CH; c += kGemmThreads) {
-            const int r = c / CH, f0 = nt * fpb + (c % CH) * 8;
-            if (r < rows && f0 < inter)
-                *reinterpret_cast<u32x4_t*>(hbuf + (int64_t)(m0 + r) * hstride + f0) =
-                    *reinterpret_cast<const u32x4_t*>(T + r * TS + (c % CH) * 8);
-        }
-    } else {
-        constexpr int TS = kBlockN + 8;
-        constexpr int CH = kBlockN / 8;
-#pragma unroll
-        for (int nj = 0; nj < kNJ; ++nj) {
-            const int nl = wv * kWaveN + nj * 32 + l32;
-            float bd = 0.f;
-            if (L.p[2].bias >= 0)
-                bd = bf2f(reinterpret_cast<const uint16_t*>(base + L.p[2].bias)[min(nt * kBlockN + nl, H - 1)]);
-#pragma unroll
-            for (int mi = 0; mi < MR; ++mi) {
-#pragma unroll
-                for (int i = 0; i < 16; ++i)
-                    T[(mi * 32 + 8 * (i >> 2) + 4 * kh + (i & 3)) * TS + nl] =
-                        __builtin_bit_cast(uint16_t, (__bf16)(acc[mi][nj][i] + bd));
-            }
-        }
-        lds_barrier();
-        for (int c = tid; c < MF * 16 * CH; c += kGemmThreads) {
-            const int r = c / CH, n0 = nt * kBlockN + (c % CH) * 8;
-            if (r < rows && n0 < H) {
-                const int d = dst_s[r];
-                uint16_t* dst = d >= 0 ? y_routed + (int64_t)d * H + n0 : y_shared + (int64_t)(-2 - d) * H + n0;
-                *reinterpret_cast<u32x4_t*>(dst) = *reinterpret_cast<const u32x4_t*>(T + r * TS + (c % CH) * 8);
-            }
-        }
-    }
-}
 
 // How a block copies its rows' scales into LDS: per row and stage one 16-bit affine scale and
 // bias, or MXFP4's two e8m0 bytes. One copy ("unit") per row is 4 bytes holding stages 2u and
@@ -419,7 +300,7 @@ __device__ __forceinline__ void pf_tile(const FwdArgs& a, const int32_t* __restr
     // loads per wave of an odd stage (A copies, B loads) and of an even stage (+ the scale copies
     // of it and the next stage, unless the tile reads its scales from the table)
     constexpr int NV1 = NA + kNJ * kBLoads<MODE>;
-    constexpr int NV0 = NV1 + ((TBL || !kScaled<MODE>) ? 0 : kAffine<MODE> ? 2 : 1);
+    constexpr int NV0 = NV1 + (TBL ? 0 : kAffine<MODE> ? 2 : 1);
     // A (and scale) copies alone, of an even and an odd stage
     constexpr int NVA1 = NA;
     constexpr int NVA0 = NV0 - kNJ * kBLoads<MODE>;
@@ -523,7 +404,7 @@ __device__ __forceinline__ void pf_tile(const FwdArgs& a, const int32_t* __restr
         // scales: paired, an even stage's slot holds its 16-bit scale (and bias) value in the
         // low half and the next stage's in the high half and an odd stage copies nothing;
         // unpaired, every stage copies its own 16 bits
-        if constexpr (TBL || !kScaled<MODE>) {
+        if constexpr (TBL) {
         } else if (spair) {
             if ((s & 1) == 0) {
                 const int gp = g & ~1;
@@ -581,7 +462,7 @@ __device__ __forceinline__ void pf_tile(const FwdArgs& a, const int32_t* __restr
     constexpr int MR = MF / 2;
     // the lane's scales of stage s, read from the ring
     // the lane's scales of one stage, as the dequantization takes them (converted once a stage):
-    // affine s 2^24 (exact) and b; MXFP4 the e8m0 scale of the stage's 32-wide group kh, which
+    // affine s kScaleUp (exact) and b; MXFP4 the e8m0 scale of the stage's 32-wide group kh, which
     // holds the lane's chunks 4 kh .. 4 kh + 3
     struct SReg {
         float s[kNJ], b[kNJ];
@@ -602,10 +483,8 @@ __device__ __forceinline__ void pf_tile(const FwdArgs& a, const int32_t* __restr
             const uint32_t sv = (*reinterpret_cast<const uint32_t*>(ss + br * 4) >> sh) & 0xFFFFu;
             if constexpr (kAffine<MODE>) {
                 const uint32_t bv = (*reinterpret_cast<const uint32_t*>(ss + ab + br * 4) >> sh) & 0xFFFFu;
-                f.s[nj] = (F16 ? h2f(sv) : bf2f(sv)) * 16777216.0f;
+                f.s[nj] = (F16 ? h2f(sv) : bf2f(sv)) * kScaleUp<MODE>;
                 f.b[nj] = F16 ? h2f(bv) : bf2f(bv);
-            } else if constexpr (!kScaled<MODE>) {
-                f.s[nj] = f.b[nj] = 0.f;      // no scales: the slot read above is not used
             } else {
                 f.s[nj] = e8m0_f32((sv >> (8 * kh)) & 0xFFu);
                 f.b[nj] = 0.f;
@@ -616,8 +495,7 @@ __device__ __forceinline__ void pf_tile(const FwdArgs& a, const int32_t* __restr
     auto deq = [&](bf16x8_t (&bop)[kNJ], const BReg& bw, const SReg& f, int kk) __attribute__((always_inline)) {
 #pragma unroll
         for (int nj = 0; nj < kNJ; ++nj) {
-            const float sv = f.s[nj], bv = f.b[nj], sc = f.s[nj];
-            bop[nj] = dq8<MODE>(bw.w[nj], kk, sv, bv, sc);
+            bop[nj] = dq8<MODE>(bw.w[nj], kk, f.s[nj], f.b[nj]);
         }
     };
 
@@ -894,10 +772,7 @@ void k_pf_gemm(FwdArgs a, const int32_t* __restrict__ order, const int32_t* __re
     const ScalePlan sp = scale_plan<MODE, KIND>(a, sh ? a.lay_sh : a.lay, K, KIND == 0 && a.act == BRX_ACT_SILU_MLP);
 #define BRX_TILE(MF, TBL) \
     pf_tile<MODE, F16, KIND, MF, TBL>(a, order, hbuf, hstride, y_routed, y_shared, ring, dst_s, e, m0, rows, ti.w, nt)
-    if constexpr (!kScaled<MODE>) {       // bf16 weights: no scales to copy
-        if (rows <= 32) BRX_TILE(2, false);
-        else BRX_TILE(4, false);
-    } else if (rows <= 32) {
+    if (rows <= 32) {
         // (32-row tiles of 4-bit codes also keep kBPairLds for their paired B loads)
         constexpr int stage_b = kBW<MODE> == 4 ? kBPairLds : 0;
         if (tile_lds<MODE>(2, true, sp.pitch) + stage_b <= kRing) BRX_TILE(2, true);
@@ -986,10 +861,12 @@ struct PfWs {
 
 inline size_t align256(size_t v) { return (v + 255) & ~(size_t)255; }
 
-// The M tile height of a kernel mode (kTileRows on the host).
+// The M tile height of a kernel mode (kTileRows on the host; kDenseRows for bf16 weights), and the
+// height its smallest scratch is counted with (what brx_moe_block_forward_noalloc accepts).
 inline int tile_rows(int mode) {
-    return mode == kModeAffine6 || mode == kModeAffine8 || mode == kModeBf16 ? 64 : kBM;
+    return mode == kModeBf16 ? kDenseRows : mode == kModeAffine6 || mode == kModeAffine8 ? 64 : kBM;
 }
+inline int scratch_rows(int mode) { return mode == kModeBf16 ? 64 : tile_rows(mode); }
 
 PfWs carve(const FwdArgs& a, int tile, void* ws) {
     const int P = a.P;
@@ -1067,7 +944,7 @@ static int thin_rows(const FwdArgs& a) {
 }
 
 // What launch_prefill cannot do without, and what it takes when it may choose.
-size_t prefill_workspace_min(const FwdArgs& a) { return carve(a, tile_rows(a.quant_mode), nullptr).bytes; }
+size_t prefill_workspace_min(const FwdArgs& a) { return carve(a, scratch_rows(a.quant_mode), nullptr).bytes; }
 
 size_t prefill_workspace_bytes(const FwdArgs& a) {
     const size_t m = prefill_workspace_min(a);
@@ -1129,7 +1006,10 @@ hipError_t launch_prefill(const FwdArgs& a, void* ws, size_t ws_bytes, int phase
         case kModeAffine6: err = BRX_GEMM(kModeAffine6); break;
         case kModeAffine8: err = BRX_GEMM(kModeAffine8); break;
         case BRX_QUANT_MXFP4: err = launch_gemm<BRX_QUANT_MXFP4, false>(a, w, E_ext, Imax, y_routed, phases, s); break;
-        case kModeBf16: err = launch_gemm<kModeBf16, false>(a, w, E_ext, Imax, y_routed, phases, s); break;
+        case kModeBf16:
+            err = launch_dense(a, ThinArgs{w.order, w.tile_start, w.tinfo, w.hbuf, y_routed, w.y_shared, E_ext, Imax,
+                                           w.mt_pad, kDenseRows}, phases, s);
+            break;
         default: err = hipErrorInvalidValue;
     }
 #undef BRX_GEMM

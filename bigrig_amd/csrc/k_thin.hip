@@ -76,7 +76,7 @@ struct Chunks {
 };
 
 // The words a lane loads a step: a quarter of its row's 128-code segment (bits words), or, for
-// bf16, its two chunks of the 64-code stage.
+// bf16, chunks g and 4 + g of the 64-code stage.
 template <int MODE>
 constexpr int kTW = kBits<MODE> == 16 ? 8 : kBits<MODE>;
 
@@ -130,61 +130,17 @@ __device__ __forceinline__ void to_chunks(const uint32_t (&w)[kTW<MODE>], Chunks
     }
 }
 
-// A stage's scale as the dequantization takes it: affine s 2^24 and b (8 bits: s and b); MXFP4
-// the e8m0 scale.
+// A chunk as an MFMA operand (s: the scale times kScaleUp, or the e8m0 scale).
 template <int MODE>
 __device__ __forceinline__ bf16x8_t chunk_ops(const uint32_t (&c)[kCW<MODE>], float s, float b) {
-    constexpr int B = kBits<MODE>;
     uint32_t o[4];
     if constexpr (kAffine<MODE>) {
-        float v[8];
-        auto lo = [&](uint32_t t, float sc) __attribute__((always_inline)) {
-            return __builtin_fmaf((float)__builtin_bit_cast(_Float16, (uint16_t)(t & 0xFFFFu)), sc, b);
-        };
-        auto hi = [&](uint32_t t, float sc) __attribute__((always_inline)) {
-            return __builtin_fmaf((float)__builtin_bit_cast(_Float16, (uint16_t)(t >> 16)), sc, b);
-        };
-        // Every value is fl(s q + b) with one rounding: a code field at bit p of a 16-bit half,
-        // alone in it and below bit 10, reads as the fp16 subnormal q 2^(p - 24), exactly, and
-        // meets s 2^(24 - p) in v_fma_mix_f32.
-        if constexpr (B == 4) {
-            const float s20 = s * 0.0625f;
-            const uint32_t u = c[0] >> 8;
-            const uint32_t t0 = c[0] & 0x000F000Fu, t1 = c[0] & 0x00F000F0u;
-            const uint32_t t2 = u & 0x000F000Fu, t3 = u & 0x00F000F0u;
-            v[0] = lo(t0, s); v[4] = hi(t0, s); v[1] = lo(t1, s20); v[5] = hi(t1, s20);
-            v[2] = lo(t2, s); v[6] = hi(t2, s); v[3] = lo(t3, s20); v[7] = hi(t3, s20);
-        } else if constexpr (B == 3) {
-            const float s21 = s * 0.125f, s18 = s * 0.015625f;
-            const uint32_t r = (c[0] & 0x1FFu) | ((c[0] << 7) & 0x01FF0000u);   // codes 0-2 | 3-5
-            const uint32_t t0 = r & 0x00070007u, t1 = r & 0x00380038u, t2 = r & 0x01C001C0u;
-            const uint32_t q = c[0] >> 18;
-            v[0] = lo(t0, s); v[3] = hi(t0, s); v[1] = lo(t1, s21); v[4] = hi(t1, s21);
-            v[2] = lo(t2, s18); v[5] = hi(t2, s18); v[6] = lo(q & 0x7u, s); v[7] = lo(q & 0x38u, s21);
-        } else if constexpr (B == 2) {
-            const float s22 = s * 0.25f, s20 = s * 0.0625f, s18 = s * 0.015625f, s16 = s * 0.00390625f;
-            const uint32_t q = c[0] >> 10;
-            v[0] = lo(c[0] & 0x3u, s); v[1] = lo(c[0] & 0xCu, s22); v[2] = lo(c[0] & 0x30u, s20);
-            v[3] = lo(c[0] & 0xC0u, s18); v[4] = lo(c[0] & 0x300u, s16);
-            v[5] = lo(q & 0x3u, s); v[6] = lo(q & 0xCu, s22); v[7] = lo(q & 0x30u, s20);
-        } else if constexpr (B == 6) {
-#pragma unroll
-            for (int i = 0; i < 8; ++i) v[i] = lo((c[i >> 2] >> (6 * (i & 3))) & 0x3Fu, s);
-        } else {
-#pragma unroll
-            for (int i = 0; i < 8; ++i)
-                v[i] = __builtin_fmaf((float)((c[i >> 2] >> (8 * (i & 3))) & 0xFFu), s, b);
-        }
-#pragma unroll
-        for (int i = 0; i < 4; ++i) o[i] = pk_bf16(v[2 * i], v[2 * i + 1]);
+        dq_affine<kBits<MODE>>(c, s, b, o);
     } else if constexpr (MODE == kModeBf16) {
 #pragma unroll
         for (int i = 0; i < 4; ++i) o[i] = c[i];
     } else {
-        o[0] = __builtin_bit_cast(uint32_t, __builtin_amdgcn_cvt_scalef32_pk_bf16_fp4(c[0], s, 0));
-        o[1] = __builtin_bit_cast(uint32_t, __builtin_amdgcn_cvt_scalef32_pk_bf16_fp4(c[0], s, 1));
-        o[2] = __builtin_bit_cast(uint32_t, __builtin_amdgcn_cvt_scalef32_pk_bf16_fp4(c[0], s, 2));
-        o[3] = __builtin_bit_cast(uint32_t, __builtin_amdgcn_cvt_scalef32_pk_bf16_fp4(c[0], s, 3));
+        dq_fp4(c[0], s, o);
     }
     return __builtin_bit_cast(bf16x8_t, u32x4_t{o[0], o[1], o[2], o[3]});
 }
@@ -243,7 +199,7 @@ __device__ __forceinline__ void thin_tile(const FwdArgs& a, const int32_t* __res
 #pragma unroll
     for (int n = 0; n < NC; ++n)
         vbw[n] = (uint32_t)mat_row(br0 + 16 * n) * (uint32_t)(K * B / 8) +
-                 (B == 16 ? 64 * (g & 1) + 16 * (g >> 1) : g * (4 * B));
+                 g * (B == 16 ? 16 : 4 * B);
     const uint32_t wbase = (uint32_t)L.p[pj].w;
     struct BReg {
         uint32_t w[NC][kTW<MODE>];
@@ -266,7 +222,7 @@ __device__ __forceinline__ void thin_tile(const FwdArgs& a, const int32_t* __res
             } else {
 #pragma unroll
                 for (int l = 0; l < kTW<MODE> / 4; ++l) {
-                    const u32x4_t v = __builtin_amdgcn_raw_buffer_load_b128(rb, vbw[n], go + (B == 16 ? 32 : 16) * l, 0);
+                    const u32x4_t v = __builtin_amdgcn_raw_buffer_load_b128(rb, vbw[n], go + (B == 16 ? 64 : 16) * l, 0);
                     q[4 * l] = v[0]; q[4 * l + 1] = v[1]; q[4 * l + 2] = v[2]; q[4 * l + 3] = v[3];
                 }
                 if constexpr (B == 6) {
@@ -359,12 +315,12 @@ __device__ __forceinline__ void thin_tile(const FwdArgs& a, const int32_t* __res
 #pragma unroll
             for (int r = 0; r < 4; ++r) acc[i][n][r] = 0.f;
 
-    // the lane's A operand addresses: chunk 4 (g & 1) + 2 j + (g >> 1) of row l16 (+ 16 m) of a
-    // stage (rows 16 apart share a swizzle key)
+    // the lane's A operand addresses: chunk 4 (g & 1) + 2 j + (g >> 1) (bf16 weights: 4 j + g, the
+    // natural order) of row l16 (+ 16 m) of a stage (rows 16 apart share a swizzle key)
     uint32_t ax[2];
 #pragma unroll
     for (int j = 0; j < 2; ++j)
-        ax[j] = (uint32_t)(l16 * 128 + (((4 * (g & 1) + 2 * j + (g >> 1)) ^ a_key(l16)) << 4));
+        ax[j] = (uint32_t)(l16 * 128 + (((B == 16 ? 4 * j + g : 4 * (g & 1) + 2 * j + (g >> 1)) ^ a_key(l16)) << 4));
     const uint8_t* const srow = tbl + br0 * ts.pitch;
     const int gs = kAffine<MODE> ? a.gshift : 0;
 
@@ -384,7 +340,7 @@ __device__ __forceinline__ void thin_tile(const FwdArgs& a, const int32_t* __res
                 if constexpr (kAffine<MODE>) {
                     const uint32_t s16 = *reinterpret_cast<const uint16_t*>(sr + 2 * (s >> gs));
                     const uint32_t b16 = *reinterpret_cast<const uint16_t*>(sr + ts.bytes + 2 * (s >> gs));
-                    sv[n] = (F16 ? h2f(s16) : bf2f(s16)) * (B == 8 ? 1.0f : 16777216.0f);
+                    sv[n] = (F16 ? h2f(s16) : bf2f(s16)) * kScaleUp<MODE>;
                     bv[n] = F16 ? h2f(b16) : bf2f(b16);
                 } else if constexpr (kScaled<MODE>) {
                     const uint32_t s16 = *reinterpret_cast<const uint16_t*>(sr + 2 * s);
