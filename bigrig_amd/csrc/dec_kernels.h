@@ -10,13 +10,13 @@
 // Gate/up, then down:
 //   k_dec_gateup1  one token: one (entry, row) item per row group; every block ranks the
 //                  token's top-k itself and block 0 records the entry table.
-//   k_dec_gateup   one token the above does not take (pairs given by the caller, more than 256
-//                  experts or three units a lane): grid (row block, entry), gate and up rows of
-//                  one expert for every pair routed to it, act() in the epilogue, h -> bf16
-//                  workspace; its blocks of row block 0 record the entry table. With the layer's
-//                  router logits given, every block ranks the top-k.
-//   k_dec_plan + k_dec_gateupT  several tokens: one block ranks and plans the step once, then one
-//                  block per (entry, row block).
+//   k_dec_gateup   several tokens with few entries and narrow experts (or one token the above
+//                  does not take): grid (row block, entry row y < 16), gate and up rows of one
+//                  expert for every token routed to it (entries y, y + 16, ...), act() in the
+//                  epilogue, h -> bf16 workspace; its blocks of row block 0 record the entry
+//                  table. With the layer's router logits given, every block ranks the top-k.
+//   k_dec_plan + k_dec_gateupT  several tokens otherwise: one block ranks and plans the step once,
+//                  then one block per (entry, row block).
 //   k_dec_down_fit / k_dec_down  grid (row block of H): down rows of every entry, each pair's
 //                  bf16 row result, and the k-ordered combine out[t] = sum_j w[t,j] * y[t,j].
 //   k_dec_downT + k_combine  after the plan: one block per (entry, row block), then the combine.
@@ -53,6 +53,7 @@ constexpr int kMaxTok = 8;
 constexpr int kMaxU = 65;     // 64 routed pairs + the shared expert
 constexpr int kXU = 144;      // LDS bytes per staged activation unit: 64 bf16 + 16 pad
 constexpr int kDownLds = 96 * 1024;   // staged h budget of the down kernel
+constexpr int kEntryRows = 16;        // block rows of the one-launch several-token gate/up kernel
 
 struct DecEntry {
     int32_t slot;             // pool slot, or -1 for the shared expert
@@ -525,10 +526,10 @@ __device__ __forceinline__ void stage_rows(const uint16_t* __restrict__ src, int
 // ------------------------------------------------------------------ gate/up
 // Wave w of the block owns rows w * RW + g (g = lane / SP, RW = 64 / SP) of the block's
 // RB = 4 RW rows, for both the gate and the up projection.
-template <int MODE, int UPL, int KP>
+template <int MODE, int UPL, int KP, bool MULTI>
 __global__ __launch_bounds__(kThreads) void k_dec_gateup(FwdArgs a, uint16_t* __restrict__ hbuf,
                                                          int hstride, DecTable* __restrict__ table,
-                                                         int lsp) {
+                                                         int lsp, int nu, int nby) {
     prefetch_args(a);
     extern __shared__ __attribute__((aligned(16))) uint8_t lds[];
     __shared__ int32_t s_e[kWave];   // P <= 64 pairs
@@ -548,80 +549,165 @@ __global__ __launch_bounds__(kThreads) void k_dec_gateup(FwdArgs a, uint16_t* __
     if constexpr (KP == 0) pe = a.pexp[min(lane, a.P - 1)];
     RouteRegs<(KP > 0 ? KP : 1)> rg;
     if constexpr (KP > 0) route_load<KP>(a, rg);
-    // every block has its entry, and x rides in the routing round trip
+    // MULTI (several tokens): most of the P + 1 possible entries are empty, so a block takes
+    // entries y, y + 16, ... and stages x only once it has one, after the routing; otherwise
+    // (one token) every block has its entry and x rides in the routing round trip
+    constexpr bool late_x = MULTI;
     StageRegs st;
     auto tok_row = [](int i) { return i; };
-    stage_issue(a.x, H, a.T, tok_row, 0, st);
+    if (!late_x) stage_issue(a.x, H, a.T, tok_row, 0, st);
     if (tid < a.E) s_g2s[tid] = g2s0;
     if (tid + kThreads < a.E) s_g2s[tid + kThreads] = g2s1;
     if constexpr (KP == 0)
         if (tid < a.P) s_e[tid] = pe;
-    stage_store<MODE>(H, a.T, 0, st, xs, xsum);
-    stage_rows<MODE>(a.x, H, a.T, tok_row, xs, xsum, kStageB);
+    if (!late_x) {
+        stage_store<MODE>(H, a.T, 0, st, xs, xsum);
+        stage_rows<MODE>(a.x, H, a.T, tok_row, xs, xsum, kStageB);
+    }
     if constexpr (KP > 0) route_rank<KP>(a, rg, s_e, blockIdx.x == 0 && blockIdx.y == 0);
     __syncthreads();
-    const int e_raw = lane < a.P ? s_e[lane] : 0;
-    Entry en;
-    int n;
-    if (!plan_entry(a, blockIdx.y, e_raw, s_g2s, en, n)) {
-        if (blockIdx.x == 0 && tid == 0) {    // no entry here: an empty table row
-            table->ent[blockIdx.y].slot = 0;
-            table->ent[blockIdx.y].nt = 0;
+    if constexpr (!MULTI) {
+        const int e_raw = lane < a.P ? s_e[lane] : 0;
+        Entry en;
+        int n;
+        if (!plan_entry(a, blockIdx.y, e_raw, s_g2s, en, n)) {
+            if (blockIdx.x == 0 && tid == 0) {    // no entry here: an empty table row
+                table->ent[blockIdx.y].slot = 0;
+                table->ent[blockIdx.y].nt = 0;
+            }
+            return;
         }
-        return;
-    }
-    if (blockIdx.x == 0 && tid == 0) {        // the entry table for the down kernel
-        DecEntry& d = table->ent[blockIdx.y];
-        d.slot = en.slot;
-        d.nt = en.nt;
-        PairIter it{en.mm, 0};
+        if (blockIdx.x == 0 && tid == 0) {        // the entry table for the down kernel
+            DecEntry& d = table->ent[blockIdx.y];
+            d.slot = en.slot;
+            d.nt = en.nt;
+            PairIter it{en.mm, 0};
+            for (int i = 0; i < en.nt; ++i) {
+                int tok;
+                d.pair[i] = it.next(a, en, tok);
+            }
+            if (blockIdx.y == 0) table->n = n;
+        }
+        const bool sh = en.e >= a.E;
+        const int inter = sh ? a.I_sh : a.I;
+        const int RW = kWave >> lsp;
+        const int r0 = blockIdx.x * kWaves * RW;
+        if (r0 >= inter) return;
+        const Layout& L = sh ? a.lay_sh : a.lay;
+        const uint8_t* base = code_base(a, en.slot);
+        const int g = lane >> lsp, sl = lane & (SP - 1);
+        const int rr = (tid >> 6) * RW + g;
+        const int row = min(r0 + rr, inter - 1);
+
+        // a two-layer expert (fc1 / fc2) has no up projection: only fc1's rows are read
+        const bool gated = a.act != BRX_ACT_SILU_MLP;
+        Units<MODE, UPL> ug, uu;
+        units_load<MODE, UPL>(base, L.p[0], row, sl, SP, a.gshift, ug);
+        if (gated) units_load<MODE, UPL>(base, L.p[1], row, sl, SP, a.gshift, uu);
+        float bg = 0.f, bu = 0.f;
+        if (L.p[0].bias >= 0) {
+            bg = bf2f(reinterpret_cast<const uint16_t*>(base + L.p[0].bias)[row]);
+            if (gated) bu = bf2f(reinterpret_cast<const uint16_t*>(base + L.p[1].bias)[row]);
+        }
+        PairIter pit{en.mm, 0};
         for (int i = 0; i < en.nt; ++i) {
             int tok;
-            d.pair[i] = it.next(a, en, tok);
-        }
-        if (blockIdx.y == 0) table->n = n;
-    }
-    const bool sh = en.e >= a.E;
-    const int inter = sh ? a.I_sh : a.I;
-    const int RW = kWave >> lsp;
-    const int r0 = blockIdx.x * kWaves * RW;
-    if (r0 >= inter) return;
-    const Layout& L = sh ? a.lay_sh : a.lay;
-    const uint8_t* base = code_base(a, en.slot);
-    const int g = lane >> lsp, sl = lane & (SP - 1);
-    const int rr = (tid >> 6) * RW + g;
-    const int row = min(r0 + rr, inter - 1);
-
-    // a two-layer expert (fc1 / fc2) has no up projection: only fc1's rows are read
-    const bool gated = a.act != BRX_ACT_SILU_MLP;
-    Units<MODE, UPL> ug, uu;
-    units_load<MODE, UPL>(base, L.p[0], row, sl, SP, a.gshift, ug);
-    if (gated) units_load<MODE, UPL>(base, L.p[1], row, sl, SP, a.gshift, uu);
-    float bg = 0.f, bu = 0.f;
-    if (L.p[0].bias >= 0) {
-        bg = bf2f(reinterpret_cast<const uint16_t*>(base + L.p[0].bias)[row]);
-        if (gated) bu = bf2f(reinterpret_cast<const uint16_t*>(base + L.p[1].bias)[row]);
-    }
-    PairIter pit{en.mm, 0};
-    for (int i = 0; i < en.nt; ++i) {
-        int tok;
-        const int pair = pit.next(a, en, tok);
-        float pg = 0.f, pu = 0.f;
-#pragma unroll
-        for (int j = 0; j < UPL; ++j) {
-            const int un = sl + SP * j;
-            if (un < U) {
-                const uint4* xu = reinterpret_cast<const uint4*>(xs + ((int64_t)tok * U + un) * kXU);
-                const float sx = kAffine<MODE> ? xsum[tok * U + un] : 0.0f;
-                pg += unit_dot<MODE, UPL>(ug, j, xu, sx, a.scale_f16);
-                if (gated) pu += unit_dot<MODE, UPL>(uu, j, xu, sx, a.scale_f16);
+            const int pair = pit.next(a, en, tok);
+            float pg = 0.f, pu = 0.f;
+    #pragma unroll
+            for (int j = 0; j < UPL; ++j) {
+                const int un = sl + SP * j;
+                if (un < U) {
+                    const uint4* xu = reinterpret_cast<const uint4*>(xs + ((int64_t)tok * U + un) * kXU);
+                    const float sx = kAffine<MODE> ? xsum[tok * U + un] : 0.0f;
+                    pg += unit_dot<MODE, UPL>(ug, j, xu, sx, a.scale_f16);
+                    if (gated) pu += unit_dot<MODE, UPL>(uu, j, xu, sx, a.scale_f16);
+                }
+            }
+            pg = group_sum(pg, SP);
+            if (gated) pu = group_sum(pu, SP);
+            if (sl == 0 && r0 + rr < inter) {
+                const float h = en.slot == kAbsentCode ? absent_nan() : act_apply(a.act, pg + bg, pu + bu, a.alpha, a.limit);
+                hbuf[(int64_t)pair * hstride + r0 + rr] = (uint16_t)f2bf(h);
             }
         }
-        pg = group_sum(pg, SP);
-        if (gated) pu = group_sum(pu, SP);
-        if (sl == 0 && r0 + rr < inter) {
-            const float h = en.slot == kAbsentCode ? absent_nan() : act_apply(a.act, pg + bg, pu + bu, a.alpha, a.limit);
-            hbuf[(int64_t)pair * hstride + r0 + rr] = (uint16_t)f2bf(h);
+    } else {
+        const int e_raw = lane < a.P ? s_e[lane] : 0;
+        // entries by, by + NB, ... (NB = the grid's rows, passed in so the kernel reads no
+        // hidden argument and its argument block stays under 512 bytes); x is staged once,
+        // with the first entry
+        const int NB = nby;
+        bool staged = false;
+        for (int u = blockIdx.y; u < nu; u += NB) {
+            Entry en;
+            int n;
+            if (!plan_entry(a, u, e_raw, s_g2s, en, n)) {
+                if (blockIdx.x == 0 && tid == 0)      // entry rows past the last: empty table rows
+                    for (int v = u; v < nu; v += NB) {
+                        table->ent[v].slot = 0;
+                        table->ent[v].nt = 0;
+                    }
+                return;
+            }
+            if (blockIdx.x == 0 && tid == 0) {        // the entry table for the down kernel
+                DecEntry& d = table->ent[u];
+                d.slot = en.slot;
+                d.nt = en.nt;
+                PairIter it{en.mm, 0};
+                for (int i = 0; i < en.nt; ++i) {
+                    int tok;
+                    d.pair[i] = it.next(a, en, tok);
+                }
+                if (u == 0) table->n = n;
+            }
+            const bool sh = en.e >= a.E;
+            const int inter = sh ? a.I_sh : a.I;
+            const int RW = kWave >> lsp;
+            const int r0 = blockIdx.x * kWaves * RW;
+            if (r0 >= inter) continue;   // uniform
+            const Layout& L = sh ? a.lay_sh : a.lay;
+            const uint8_t* base = code_base(a, en.slot);
+            const int g = lane >> lsp, sl = lane & (SP - 1);
+            const int rr = (tid >> 6) * RW + g;
+            const int row = min(r0 + rr, inter - 1);
+
+            const bool gated = a.act != BRX_ACT_SILU_MLP;
+            Units<MODE, UPL> ug, uu;
+            units_load<MODE, UPL>(base, L.p[0], row, sl, SP, a.gshift, ug);
+            if (gated) units_load<MODE, UPL>(base, L.p[1], row, sl, SP, a.gshift, uu);
+            float bg = 0.f, bu = 0.f;
+            if (L.p[0].bias >= 0) {
+                bg = bf2f(reinterpret_cast<const uint16_t*>(base + L.p[0].bias)[row]);
+                if (gated) bu = bf2f(reinterpret_cast<const uint16_t*>(base + L.p[1].bias)[row]);
+            }
+            if (!staged) {   // the weights are in flight
+                stage_dense<MODE>(a.x, H, a.T, tok_row, xs, xsum);
+                __syncthreads();
+                staged = true;
+            }
+            PairIter pit{en.mm, 0};
+            for (int i = 0; i < en.nt; ++i) {
+                int tok;
+                const int pair = pit.next(a, en, tok);
+                float pg = 0.f, pu = 0.f;
+    #pragma unroll
+                for (int j = 0; j < UPL; ++j) {
+                    const int un = sl + SP * j;
+                    if (un < U) {
+                        const uint4* xu = reinterpret_cast<const uint4*>(xs + ((int64_t)tok * U + un) * kXU);
+                        const float sx = kAffine<MODE> ? xsum[tok * U + un] : 0.0f;
+                        pg += unit_dot<MODE, UPL>(ug, j, xu, sx, a.scale_f16);
+                        if (gated) pu += unit_dot<MODE, UPL>(uu, j, xu, sx, a.scale_f16);
+                    }
+                }
+                pg = group_sum(pg, SP);
+                if (gated) pu = group_sum(pu, SP);
+                if (sl == 0 && r0 + rr < inter) {
+                    const float h = en.slot == kAbsentCode ? absent_nan()
+                                                           : act_apply(a.act, pg + bg, pu + bu, a.alpha, a.limit);
+                    hbuf[(int64_t)pair * hstride + r0 + rr] = (uint16_t)f2bf(h);
+                }
+            }
         }
     }
 }
@@ -1420,11 +1506,19 @@ template <int MODE, int UPL>
 hipError_t launch_gateup(const FwdArgs& a, uint16_t* hbuf, DecTable* table, int nu, int Imax, int SP,
                          hipStream_t s) {
     const int RB = kWaves * (kWave / SP);
-    dim3 grid((Imax + RB - 1) / RB, nu), block(kThreads);
+    // entry rows: one per block row up to 16; past that (several tokens, where most of the
+    // P + 1 possible entries are empty) a block takes entries y, y + 16, ...
+    dim3 grid((Imax + RB - 1) / RB, a.T > 1 && nu > kEntryRows ? kEntryRows : nu), block(kThreads);
     // staged x of up to T tokens
     const size_t lds = (size_t)a.T * (a.H / 64) * (kXU + 4);
     const int lsp = __builtin_ctz(SP);
-#define BRX_GU(KP) hipLaunchKernelGGL((k_dec_gateup<MODE, UPL, KP>), grid, block, lds, s, a, hbuf, Imax, table, lsp)
+#define BRX_GU(KP)                                                                                     \
+    do {                                                                                               \
+        if (a.T > 1)                                                                                   \
+            hipLaunchKernelGGL((k_dec_gateup<MODE, UPL, KP, true>), grid, block, lds, s, a, hbuf, Imax, table, lsp, nu, (int)grid.y); \
+        else                                                                                           \
+            hipLaunchKernelGGL((k_dec_gateup<MODE, UPL, KP, false>), grid, block, lds, s, a, hbuf, Imax, table, lsp, nu, (int)grid.y); \
+    } while (0)
     if (!a.logits) BRX_GU(0);
     else if (a.E <= 64) BRX_GU(1);
     else if (a.E <= 128) BRX_GU(2);
@@ -1549,18 +1643,22 @@ hipError_t launch_mode(const FwdArgs& a, uint16_t* hbuf, DecTable* table, uint16
     const int PT = P + (a.auto_shared ? a.T : 0);
     const int nu = P + (a.auto_shared ? 1 : 0);
     const int Imax = a.I > a.I_sh ? a.I : a.I_sh;
-    // Several tokens: the plan launch, then one block per (entry, rows). (Up to 32 possible entries
-    // once took one launch in which every block ranked and planned the step and the down kernel
-    // staged every pair's h rows; per layer, before and after: 3 tokens of 64 4-bit experts 49.2 ->
-    // 42.4 us, 2 and 4 tokens of the Qwen3 shape 31.7 -> 29.6 and 47.9 -> 35.2, 2, 4 and 8 of the
-    // gpt-oss shape 48.9 -> 41, 95.6 -> 58 and 185.8 -> 88, 2 and 3 of 256 experts 26.8 -> 26.5 and
-    // 32.4 -> 29.5.)
-    const bool per_entry = a.T > 1;
+    // Several tokens: either the plan launch, one block per (entry, rows) for each projection and the
+    // combine (five launches with the router), or one launch in which every gate/up block ranks and
+    // plans the step itself and a down kernel that stages every pair's h rows and combines (three).
+    // The first wins with many entries or much to multiply, the second where the two launches
+    // saved matter more. Three / five launches, us a layer: 2 tokens (16 entries) at H x I 2048 x 512
+    // 23.8 / 26.3, 2048 x 768 31.9 / 29.6; 3 tokens (24) at 1024 x 768 25.5 / 26.0, 2048 x 512 30.6 / 29.4,
+    // 2048 x 1024 49.2 / 42.4; 4 tokens (32) at 768 x 512 29.2 / 27.9, 2048 x 768 47.9 / 35.2; top-4 MXFP4 at
+    // 4 tokens (16) 1024 x 768 20.2 / 22.3, 2880 x 2880 95.6 / 58, at 8 tokens (32) 768 x 512 28.9 / 24.5 and
+    // 2880 x 2880 186 / 88. So the line: 32 entries, or 20 M weights a projection over the entries.
+    const bool per_entry = a.T > 1 && (nu >= 2 * kEntryRows || (int64_t)nu * a.H * Imax >= 20 * 1000 * 1000);
     // one token: one unit per lane where the row allows it (twice the waves of two units per
     // lane, each with half the dequant-dot work and far fewer registers: 11.1 -> 10.2 us per
     // layer on H = 2048); several tokens: two units per lane, half the blocks, each staging
-    // x once for twice the rows. The split fixes each row's summation order and
-    // depends on the widths alone: a step's rows do not depend on how many pairs share its launch (a pool's span calls against the whole step).
+    // x once for twice the rows. The split fixes each row's summation order, so both
+    // several-token kernels take the same one: a step's rows do not depend on how many
+    // pairs share its launch (a pool's span calls against the whole step).
     int SPg, uplg;
     pick_split(a.H / 64, a.T > 1 && kMaxUpl<MODE> > 2 ? 2 : 1, SPg, uplg, kMaxUpl<MODE>);
     // the one-token gate/up kernel makes every pair its own entry (pairs given by the caller may
@@ -1589,8 +1687,8 @@ hipError_t launch_mode(const FwdArgs& a, uint16_t* hbuf, DecTable* table, uint16
         hipError_t err;
         // (the same split for both down kernels, as for gate/up)
         pick_split(Imax / 64, kMaxUpl<MODE> > 2 ? 3 : 1, SP, upl_, kMaxUpl<MODE>);
-        // several tokens: one block per (entry, rows), then the combine; one token: every block
-        // stages every pair's h rows and combines in its epilogue
+        // the per-entry form: one block per (entry, rows), then the combine; else every block stages
+        // every pair's h rows and combines in its epilogue
         if (per_entry) {
             uint16_t* yr = a.yun ? a.yun : y_routed;
             err = [&]() -> hipError_t { BRX_UPL_CASES(launch_downT, a, hbuf, table, nu, Imax, SP, yr, y_shared, s); }();
