@@ -40,9 +40,12 @@ DECODE_MAX_PAIRS = 64
 
 
 def _stream(stream=None):
+    """The raw handle of `stream`, or of the current device's current stream (read without building a
+    torch Stream object: 0.4 instead of 2.7 us a call)."""
+    if stream is not None:
+        return stream.cuda_stream
     import torch
-    s = stream if stream is not None else torch.cuda.current_stream()
-    return s.cuda_stream
+    return torch._C._cuda_getCurrentRawStream(torch._C._cuda_getDevice())
 
 
 def _dptr(t) -> int | None:
@@ -59,7 +62,7 @@ def router_topk(spec: LayerSpec, x, w_router, bias=None, shared_gate_w=None, str
     idx = torch.empty((T, spec.top_k), dtype=torch.int32, device=dev)
     w = torch.empty((T, spec.top_k), dtype=torch.float32, device=dev)
     sg = torch.empty(T, dtype=torch.float32, device=dev) if shared_gate_w is not None else None
-    d = spec.desc()
+    d = spec.c_desc
     L.check(L.load().brx_router_topk(C.byref(d), _dptr(x2), _dptr(w_router), _dptr(bias),
                                      _dptr(shared_gate_w), T, _dptr(idx), _dptr(w), _dptr(sg),
                                      _stream(stream)))
@@ -75,7 +78,7 @@ def path_flag(n_tokens: int, top_k: int) -> int:
 
 def moe_forward(spec: LayerSpec, pool: ExpertPool, x2, idx, w=None, shared=None, sgate=None,
                 out=None, y_unreduced=None, flags=None, stream=None):
-    d = spec.desc()
+    d = spec.c_desc
     T = x2.shape[0]
     L.check(L.load().brx_moe_forward(
         C.byref(d), pool.device.handle, _dptr(x2), _dptr(idx), _dptr(w), _dptr(shared),
@@ -92,7 +95,7 @@ def moe_block(spec: LayerSpec, pool: ExpertPool, x2, router_w, router_bias=None,
     T = x2.shape[0]
     if out is None:
         out = torch.empty((T, spec.hidden), dtype=torch.bfloat16, device=x2.device)
-    d = spec.desc()
+    d = spec.c_desc
     L.check(L.load().brx_moe_block_forward(
         C.byref(d), pool.device.handle, _dptr(x2), _dptr(router_w), _dptr(router_bias),
         _dptr(shared_gate_w), _dptr(shared), T, _dptr(out), _dptr(out_idx), _dptr(out_w), flags,
@@ -102,7 +105,7 @@ def moe_block(spec: LayerSpec, pool: ExpertPool, x2, router_w, router_bias=None,
 
 def forward_pairs(spec: LayerSpec, pool: ExpertPool, x2, pair_tok, pair_exp, pair_row, y_rows,
                   flags: int, shared=None, stream=None):
-    d = spec.desc()
+    d = spec.c_desc
     L.check(L.load().brx_moe_forward_pairs(
         C.byref(d), pool.device.handle, _dptr(x2), x2.shape[0], _dptr(pair_tok), _dptr(pair_exp),
         _dptr(pair_row), pair_exp.numel(), y_rows.shape[0], _dptr(shared), _dptr(y_rows), flags,
@@ -110,7 +113,7 @@ def forward_pairs(spec: LayerSpec, pool: ExpertPool, x2, pair_tok, pair_exp, pai
 
 
 def combine(spec: LayerSpec, y_routed, w, out, y_shared=None, sgate=None, stream=None):
-    d = spec.desc()
+    d = spec.c_desc
     L.check(L.load().brx_combine(C.byref(d), _dptr(y_routed), _dptr(w), _dptr(y_shared),
                                  _dptr(sgate), w.shape[0], _dptr(out), _stream(stream)))
 
@@ -120,7 +123,7 @@ def dequant(spec: LayerSpec, expert_dev, proj: int, shared: bool = False, stream
     inter = spec.shared_inter if shared else spec.inter
     n_out, n_in = (inter, spec.hidden) if proj < 2 else (spec.hidden, inter)
     out = torch.empty((n_out, n_in), dtype=torch.float32, device=expert_dev.device)
-    d = spec.desc()
+    d = spec.c_desc
     L.check(L.load().brx_dequant(C.byref(d), _dptr(expert_dev), proj, int(shared), _dptr(out),
                                  _stream(stream)))
     return out
@@ -131,7 +134,7 @@ def sort_pairs(spec: LayerSpec, idx, stream=None):
     T = idx.shape[0]
     order = torch.empty(T * spec.top_k, dtype=torch.int32, device=idx.device)
     offsets = torch.empty(spec.n_experts + 1, dtype=torch.int32, device=idx.device)
-    d = spec.desc()
+    d = spec.c_desc
     L.check(L.load().brx_sort_pairs(C.byref(d), _dptr(idx), T, _dptr(order), _dptr(offsets),
                                     _stream(stream)))
     return order, offsets
@@ -206,7 +209,7 @@ class StreamingSwitchGLU:
         or, host-served, the admissions decided from the routing that has come back since."""
         if self._serve is not None:
             self._serve.service(stream)
-        else:
+        elif self._pool.table_stale:
             self._pool.g2s_device(_stream(stream))
 
     def _after(self, idx, stream=None) -> None:

@@ -437,6 +437,11 @@ class ExpertPool:
         """Every expert resident, so no request can miss (stream.py:782-789)."""
         return self.capacity == self.n_experts and self.resident == self.n_experts
 
+    @property
+    def table_stale(self) -> bool:
+        """Residency changed since the table was last uploaded (g2s_device)."""
+        return self._table_stale
+
     def g2s_device(self, stream) -> None:
         """Upload the table when residency changed (stream.py:791-797); stream-ordered."""
         if self._table_stale and not self.host_served:

@@ -107,6 +107,11 @@ class LayerSpec:
                          _RDT[self.router_dtype], self.shared_inter, self.n_group,
                          self.topk_group, self.route_scale)
 
+    @functools.cached_property
+    def c_desc(self):
+        """desc(), built once: the descriptor the library's calls read (it is never written)."""
+        return self.desc()
+
 
 # The synthetic layer shapes the benchmarks and parity tests run (hidden, experts, top-k,
 # intermediate, routing rule, quantization).
