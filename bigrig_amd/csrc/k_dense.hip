@@ -15,6 +15,7 @@
 // the bytes (128 rows, 32-K stages: 371 + 255 us). The general kernel's 64-row tiles, whose lanes
 // loaded their own B operands, took 567 + 306.
 #include "pf_common.h"
+#include "stage_addr.h"
 
 namespace brx {
 namespace {
@@ -69,10 +70,9 @@ __device__ __forceinline__ void dense_tile(const FwdArgs& a, const int32_t* __re
 #pragma unroll
     for (int i = 0; i < NA; ++i) {
         const int rl = copy_of(i) * 8 + (lane >> 3), r = min(rl, rows - 1);
-        const int c = (lane & 7) ^ a_key(rl);
         const uint32_t row = KIND == 0 ? (uint32_t)pair_token(a, order[m0 + r]) * (uint32_t)(H * 2)
                                        : (uint32_t)(m0 + r) * (uint32_t)(hstride * 2);
-        va[i] = rl >= rows ? a_bytes : row + c * 16;
+        va[i] = a_lane_offset(rl, rows, row, (lane & 7) ^ a_key(rl), a_bytes);
     }
     // ---- B: LDS row 64 n + 32 j + q is column q of fragment j of the waves wn = n. KIND 0: fragment
     // 0 is 32 gate rows (nt * 128 + 32 n + q), fragment 1 the same features' up rows; a two-layer
@@ -102,16 +102,17 @@ __device__ __forceinline__ void dense_tile(const FwdArgs& a, const int32_t* __re
     // a stage past the last is issued through descriptors of no bytes, so the waits count the same
     // copies throughout
     auto issue = [&](int s, int at) __attribute__((always_inline)) {
-        const bool in = s < nst;
-        const __amdgpu_buffer_rsrc_t ra = make_rsrc(KIND == 0 ? (const void*)a.x : (const void*)hbuf, in ? a_bytes : 0u);
-        const __amdgpu_buffer_rsrc_t rb = make_rsrc(base, in ? (uint32_t)L.bytes : 0u);
+        const StageSrc sa = stage_src(s, nst, a_bytes, (uint32_t)s * 128u);
+        const StageSrc sb = stage_src(s, nst, (uint32_t)L.bytes, (uint32_t)s * 128u);
+        const __amdgpu_buffer_rsrc_t ra = make_rsrc(KIND == 0 ? (const void*)a.x : (const void*)hbuf, sa.records);
+        const __amdgpu_buffer_rsrc_t rb = make_rsrc(base, sb.records);
         uint8_t* st = ring + at * STAGE;
 #pragma unroll
         for (int i = 0; i < NB; ++i)
-            __builtin_amdgcn_raw_ptr_buffer_load_lds(rb, (LDS_PTR)(st + (wv * NB + i) * 1024), 16, vb[i], s * 128, 0, 0);
+            __builtin_amdgcn_raw_ptr_buffer_load_lds(rb, (LDS_PTR)(st + (wv * NB + i) * 1024), 16, vb[i], sb.soffset, 0, 0);
 #pragma unroll
         for (int i = 0; i < NA; ++i)
-            __builtin_amdgcn_raw_ptr_buffer_load_lds(ra, (LDS_PTR)(st + kDB + copy_of(i) * 1024), 16, va[i], s * 128, 0, 0);
+            __builtin_amdgcn_raw_ptr_buffer_load_lds(ra, (LDS_PTR)(st + kDB + copy_of(i) * 1024), 16, va[i], sa.soffset, 0, 0);
         asm volatile("" ::: "memory");
     };
 #pragma unroll

@@ -23,11 +23,11 @@
 #include <type_traits>
 
 #include "pf_common.h"
+#include "stage_addr.h"
 
 namespace brx {
 namespace {
 
-constexpr int kTWaves = 4;
 constexpr int kTThreads = 64 * kTWaves;
 // weight rows per block (16 NC a wave) and floats between rows of the output tile in LDS
 template <int NC>
@@ -156,8 +156,7 @@ __device__ __forceinline__ void thin_tile(const FwdArgs& a, const int32_t* __res
     constexpr int SG = kTSG<MODE>, NR = kTNR<MODE, MQ>;
     constexpr int SAst = 16 * MQ * 128;            // A bytes of a stage
     constexpr int SA = SG * SAst;                  // ... of a step
-    constexpr int NCH = SA / 1024;                 // 1 KB A copies a step, NA of them a wave
-    constexpr int NA = (NCH + kTWaves - 1) / kTWaves;
+    constexpr int NA = kTAWave<SG, MQ>;            // 1 KB A copies of a wave and step
     constexpr int LPC = B == 16 || B == 6 || B == 8 ? 2 : 1;   // loads per column fragment and step
     constexpr int NV = NA + NC * LPC;
     const bool sh = e >= a.E;
@@ -177,13 +176,11 @@ __device__ __forceinline__ void thin_tile(const FwdArgs& a, const int32_t* __res
     // requested under it
     const uint32_t a_bytes = KIND == 0 ? (uint32_t)((int64_t)a.T * H * 2)
                                        : (uint32_t)((int64_t)(m0 + rows) * hstride * 2);
-    // copy i of this wave (the waves past the last copy of a small stage repeat it)
-    auto chunk_of = [&](int i) __attribute__((always_inline)) { return min(wv * NA + i, NCH - 1); };
     int pr[NA];
     if constexpr (KIND == 0) {
 #pragma unroll
         for (int i = 0; i < NA; ++i) {
-            const int rl = ((chunk_of(i) * 64 + lane) >> 3) % (16 * MQ);
+            const int rl = thin_a_row<SG, MQ>(wv, i, lane);
             pr[i] = order[m0 + min(rl, rows - 1)];
         }
     }
@@ -198,8 +195,7 @@ __device__ __forceinline__ void thin_tile(const FwdArgs& a, const int32_t* __res
     uint32_t vbw[NC];
 #pragma unroll
     for (int n = 0; n < NC; ++n)
-        vbw[n] = (uint32_t)mat_row(br0 + 16 * n) * (uint32_t)(K * B / 8) +
-                 g * (B == 16 ? 16 : 4 * B);
+        vbw[n] = thin_b_lane(B, K, (uint32_t)mat_row(br0 + 16 * n), g);
     const uint32_t wbase = (uint32_t)L.p[pj].w;
     struct BReg {
         uint32_t w[NC][kTW<MODE>];
@@ -207,9 +203,11 @@ __device__ __forceinline__ void thin_tile(const FwdArgs& a, const int32_t* __res
     // Steps past the last are issued like the others, through a descriptor of no bytes (the range
     // check answers without memory traffic): every wait below then counts the same loads, also
     // the compiler's own for the B registers, which would drain the counter after a guarded load.
+    // An odd last stage's step reads on past the row, into the next row or the matrix's scales.
     auto issue_b = [&](int p, BReg& r) __attribute__((always_inline)) {
-        const __amdgpu_buffer_rsrc_t rb = make_rsrc(base, p < nsteps ? (uint32_t)L.bytes : 0u);
-        const uint32_t go = wbase + (uint32_t)p * (8 * B * SG);
+        const StageSrc src = stage_src(p, nsteps, (uint32_t)L.bytes, wbase + thin_b_step(B, SG, p));
+        const __amdgpu_buffer_rsrc_t rb = make_rsrc(base, src.records);
+        const uint32_t go = src.soffset;
 #pragma unroll
         for (int n = 0; n < NC; ++n) {
             uint32_t* q = r.w[n];
@@ -222,11 +220,11 @@ __device__ __forceinline__ void thin_tile(const FwdArgs& a, const int32_t* __res
             } else {
 #pragma unroll
                 for (int l = 0; l < kTW<MODE> / 4; ++l) {
-                    const u32x4_t v = __builtin_amdgcn_raw_buffer_load_b128(rb, vbw[n], go + (B == 16 ? 64 : 16) * l, 0);
+                    const u32x4_t v = __builtin_amdgcn_raw_buffer_load_b128(rb, vbw[n] + (B == 16 ? 64 : 16) * l, go, 0);
                     q[4 * l] = v[0]; q[4 * l + 1] = v[1]; q[4 * l + 2] = v[2]; q[4 * l + 3] = v[3];
                 }
                 if constexpr (B == 6) {
-                    const u32x2_t v = __builtin_amdgcn_raw_buffer_load_b64(rb, vbw[n], go + 16, 0);
+                    const u32x2_t v = __builtin_amdgcn_raw_buffer_load_b64(rb, vbw[n] + 16, go, 0);
                     q[4] = v[0]; q[5] = v[1];
                 }
             }
@@ -274,13 +272,11 @@ __device__ __forceinline__ void thin_tile(const FwdArgs& a, const int32_t* __res
     uint32_t va[NA];
 #pragma unroll
     for (int i = 0; i < NA; ++i) {
-        const int ci = chunk_of(i) * 64 + lane;
-        const int sub = ci / (SAst / 16), rl = (ci >> 3) % (16 * MQ);
-        const int c = (ci & 7) ^ a_key(rl);
+        const int rl = thin_a_row<SG, MQ>(wv, i, lane);
         const uint32_t row = KIND == 0 ? (uint32_t)pair_token(a, pr[i]) * (uint32_t)(H * 2)
                                        : (uint32_t)(m0 + min(rl, rows - 1)) * (uint32_t)(hstride * 2);
         // rows past the tile's pairs: from past the buffer's end (zeros, no cache access)
-        va[i] = rl >= rows ? a_bytes : row + sub * 128 + c * 16;
+        va[i] = a_lane_offset(rl, rows, row, (lane & 7) ^ a_key(rl), a_bytes);
     }
     if constexpr (KIND == 1) {
         if (tid < 16 * MQ) {
@@ -294,12 +290,13 @@ __device__ __forceinline__ void thin_tile(const FwdArgs& a, const int32_t* __res
     }
     auto issue_a = [&](int p) __attribute__((always_inline)) {
         uint8_t* st = smem + (p % NR) * SA;
-        const __amdgpu_buffer_rsrc_t ra =
-            make_rsrc(KIND == 0 ? (const void*)a.x : (const void*)hbuf, p < nsteps ? a_bytes : 0u);
+        const int q = p * SG + thin_a_stage<SG, MQ>(wv);
+        const StageSrc src = stage_src(q, nst, a_bytes, (uint32_t)q * 128u);
+        const __amdgpu_buffer_rsrc_t ra = make_rsrc(KIND == 0 ? (const void*)a.x : (const void*)hbuf, src.records);
 #pragma unroll
         for (int i = 0; i < NA; ++i)
-            __builtin_amdgcn_raw_ptr_buffer_load_lds(ra, (LDS_PTR)(st + chunk_of(i) * 1024), 16, va[i],
-                                                     p * (SG * 128), 0, 0);
+            __builtin_amdgcn_raw_ptr_buffer_load_lds(ra, (LDS_PTR)(st + thin_a_copy<SG, MQ>(wv, i) * 1024), 16, va[i],
+                                                     src.soffset, 0, 0);
     };
 #pragma unroll
     for (int t = 0; t < NR - 1; ++t) issue_a(t);
