@@ -6,8 +6,10 @@
 // (96 of the 128 bytes a clock LDS gives at the full MFMA rate). There is nothing to dequantize, so
 // both operands are copied straight into LDS by the buffer unit in 64-K stages: whole 128-byte lines
 // (32-K stages, half a line at a time, took 389 + 273 us where these take 355 + 253: each line
-// crossed from L2 twice). K runs in its natural order, 16 a MFMA, as in k_thin.hip's bf16 form: same
-// bits.
+// crossed from L2 twice). A 64-K stage is summed in the order of the other grouped GEMMs, chunks kk and
+// 4 + kk (8 K each) in MFMA kk, so a row has the same bits from this kernel and from k_thin.hip, and
+// those its exactly representable quantized weights give; the operands come from LDS, where any
+// order costs the same.
 //
 // Bound (4096 tokens of the Qwen3 shape, gate/up 355 us, of which the MFMAs alone are 117, the copies
 // alone 182 and a tile's start, barriers and epilogue 123): the copies, then the start and end of a
@@ -126,10 +128,10 @@ __device__ __forceinline__ void dense_tile(const FwdArgs& a, const int32_t* __re
 #pragma unroll
             for (int r = 0; r < 16; ++r) acc[i][j][r] = 0.f;
 
-    // operand addresses of MFMA kk: chunk 2 kk + kh of row l32 (+ 32 m: the same key)
+    // operand addresses of MFMA kk: chunk 4 kh + kk of row l32 (+ 32 m: the same key)
     uint32_t ad[4];
 #pragma unroll
-    for (int kk = 0; kk < 4; ++kk) ad[kk] = (uint32_t)(l32 * 128 + (((2 * kk + kh) ^ a_key(l32)) << 4));
+    for (int kk = 0; kk < 4; ++kk) ad[kk] = (uint32_t)(l32 * 128 + (((4 * kh + kk) ^ a_key(l32)) << 4));
     const bool active = wm < WM;   // uniform
 
     int at = 0, next = NS - 1;

@@ -67,6 +67,14 @@ __device__ __forceinline__ void swap32(uint32_t& v0, uint32_t& v1) {
     v1 = p[1];
 }
 
+// The same for the 16-lane groups: v0 = (v0 of groups 0 and 2) with v1's of the same two after each,
+// v1 = (v0 of groups 1 and 3) with v1's of the same two after each.
+__device__ __forceinline__ void swap16(uint32_t& v0, uint32_t& v1) {
+    const auto p = __builtin_amdgcn_permlane16_swap(v0, v1, false, false);
+    v0 = p[0];
+    v1 = p[1];
+}
+
 // A lane's codes of one step: chunk (8 codes) j of stage t in c[t][j], as chunk_ops takes them.
 template <int MODE>
 constexpr int kCW = kBits<MODE> == 16 ? 4 : kBits<MODE> >= 6 ? 2 : 1;   // words a chunk
@@ -76,22 +84,27 @@ struct Chunks {
 };
 
 // The words a lane loads a step: a quarter of its row's 128-code segment (bits words), or, for
-// bf16, chunks g and 4 + g of the 64-code stage.
+// bf16, a chunk of each half of the 64-code stage (chunks 0, 2, 1, 3 of it for lane groups 0 to 3).
 template <int MODE>
 constexpr int kTW = kBits<MODE> == 16 ? 8 : kBits<MODE>;
 
 // A step's chunks from the quarter q = 2 t + h of the row segment that lane group q loaded: it
 // holds chunks 4 h + 2 j + b of stage t, while the MFMA order gives group 2 b + h chunks
 // 4 h + 2 j + b of both stages. So the lane halves trade t for b: one v_permlane32_swap a word
-// pair.
+// pair. A bf16 lane group holds chunks i and 4 + i of one stage, and groups 2 b and 2 b + 1 trade in
+// the same way (v_permlane16_swap): loads of chunks 4 (g & 1) + 2 j + (g >> 1) straight into place
+// would read 32 bytes of a row at a time instead of 64.
 template <int MODE>
 __device__ __forceinline__ void to_chunks(const uint32_t (&w)[kTW<MODE>], Chunks<MODE>& o) {
     constexpr int B = kBits<MODE>;
     if constexpr (B == 16) {
 #pragma unroll
-        for (int j = 0; j < 2; ++j)
-#pragma unroll
-            for (int i = 0; i < 4; ++i) o.c[0][j][i] = w[4 * j + i];
+        for (int i = 0; i < 4; ++i) {
+            uint32_t a = w[i], b = w[4 + i];
+            swap16(a, b);
+            o.c[0][0][i] = a;
+            o.c[0][1][i] = b;
+        }
     } else if constexpr (B == 2) {
         // word j holds chunks b = 0 and 1 in its halves: both lanes of a pair take the word of
         // stage 0's lane and that of stage 1's, and shift their own half down
@@ -312,12 +325,12 @@ __device__ __forceinline__ void thin_tile(const FwdArgs& a, const int32_t* __res
 #pragma unroll
             for (int r = 0; r < 4; ++r) acc[i][n][r] = 0.f;
 
-    // the lane's A operand addresses: chunk 4 (g & 1) + 2 j + (g >> 1) (bf16 weights: 4 j + g, the
-    // natural order) of row l16 (+ 16 m) of a stage (rows 16 apart share a swizzle key)
+    // the lane's A operand addresses: chunk 4 (g & 1) + 2 j + (g >> 1) of row l16 (+ 16 m) of a stage
+    // (rows 16 apart share a swizzle key)
     uint32_t ax[2];
 #pragma unroll
     for (int j = 0; j < 2; ++j)
-        ax[j] = (uint32_t)(l16 * 128 + (((B == 16 ? 4 * j + g : 4 * (g & 1) + 2 * j + (g >> 1)) ^ a_key(l16)) << 4));
+        ax[j] = (uint32_t)(l16 * 128 + ((4 * (g & 1) + 2 * j + (g >> 1)) ^ a_key(l16)) * 16);
     const uint8_t* const srow = tbl + br0 * ts.pitch;
     const int gs = kAffine<MODE> ? a.gshift : 0;
 

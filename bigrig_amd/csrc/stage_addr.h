@@ -52,9 +52,10 @@ constexpr int thin_a_stage(int wv) {
 }
 
 // B loads of a thin step of `bits`-bit weights (16: bf16): lane group g's first load of weight row
-// `row` (K inputs), and the scalar offset of step p in the matrix.
+// `row` (K inputs; bf16 groups 0 to 3 start at chunks 0, 2, 1 and 3), and the scalar offset of step p
+// in the matrix.
 constexpr uint32_t thin_b_lane(int bits, int K, uint32_t row, int g) {
-    return row * (uint32_t)(K * bits / 8) + (uint32_t)(g * (bits == 16 ? 16 : 4 * bits));
+    return row * (uint32_t)(K * bits / 8) + (uint32_t)(bits == 16 ? 16 * (2 * (g & 1) + (g >> 1)) : 4 * bits * g);
 }
 constexpr uint32_t thin_b_step(int bits, int SG, int p) { return (uint32_t)p * (uint32_t)(8 * bits * SG); }
 

@@ -5,12 +5,15 @@ oracle and the float64 truth (a shared expert, biases, a two-layer expert, a par
 tile); the whole block with its routing bit-exact and the same bits as router + operator; a
 bounded pool bit-identical to full residency; a bf16 checkpoint served through a bounded pool.
 The full-size Qwen3-30B-A3B-bf16 layer runs in test_gpu_full_size.py."""
+from dataclasses import replace
+
 import numpy as np
 import pytest
 
 import oracle
 from bigrig_amd import formats as F
 from bigrig_amd import layer as ops
+from bigrig_amd import lib as L
 from bigrig_amd.spec import E256_SHARED, QWEN3_30B_A3B
 from tests.gpu_util import bits, build_gpu_layer, bytes_dev, to_dev_bits
 from tests.helpers import make_layer, make_x, small
@@ -151,3 +154,66 @@ def test_bf16_checkpoint_bounded_pool(gpu, tmp_path):
         assert r < TOL, f"T={T}: rel L2 {r:.3e}"
     assert pool.admits > C
     pool.close()
+
+
+def _bf16_copy(lay):
+    """The layer with its MXFP4 experts' weights, which bf16 holds exactly, unquantized."""
+    spec = lay.spec
+    wide = replace(spec, quant=QN)
+    def conv(blob):
+        sp = spec.expert_spec()
+        arr = F.split_expert(blob, sp)
+        out = b""
+        for p in sp:
+            w = F.dequantize_projection(arr, p, spec.quant)
+            b = F.f32_to_bf16_bits(w)
+            assert np.array_equal(F.bf16_bits_to_f32(b), w)
+            out += b.tobytes()
+            if (p, "bias") in arr:
+                out += np.ascontiguousarray(arr[(p, "bias")]).tobytes()
+        assert len(out) == wide.bytes_per_expert
+        return out
+    return replace(lay, spec=wide, experts=[conv(e) for e in lay.experts])
+
+
+DENSE_RUNS = [300, 256, 257, 129, 128, 127, 65, 64, 33, 32, 31, 1, 0, 7, 100, 200]   # tiles of 32 to 256 rows
+THIN_RUNS = [1, 15, 16, 17, 31, 32, 33, 63, 64, 65, 100, 0, 2, 7, 0, 3]               # 64-row tiles, 128-row blocks
+FEW_RUNS = [1, 15, 16, 17, 2, 0, 3, 0, 1, 0, 0, 2, 0, 0, 0, 1]                        # 64-row blocks
+
+
+@pytest.mark.parametrize("runs", [DENSE_RUNS, THIN_RUNS, FEW_RUNS, [min(r, 16) for r in FEW_RUNS]],
+                         ids=["dense", "thin", "thin-few", "thin-few16"])
+@pytest.mark.parametrize("kw", [dict(hidden=1536, inter=768), dict(hidden=576, inter=192, has_bias=True,
+                                                                 act="swiglu_clamped"),
+                                dict(hidden=64, inter=64), dict(hidden=320, inter=448, act="silu_mlp")],
+                         ids=["1536x768", "576x192-clamped", "64x64", "320x448-mlp"])
+def test_bf16_rows_are_the_exactly_quantized_rows(gpu, kw, runs):
+    """MXFP4 weights are exact in bf16, and every grouped GEMM sums a row over K in one order: the
+    bf16 kernels give the bits the 4-bit kernels give for the same weights, in tiles of every height."""
+    import torch
+    E = len(runs)
+    spec = small(QWEN3_30B_A3B, n_experts=E, top_k=2, quant=F.QuantSpec(4, 32, "mxfp4"), **kw)
+    lay = make_layer(spec, seed=890)
+    T = min(max(runs), 64)
+    xd = to_dev_bits(make_x(T, spec.hidden, seed=891), gpu)
+    pexp = np.repeat(np.arange(E, dtype=np.int32), runs)
+    ptok = np.concatenate([(np.arange(r) * 3 + e) % T for e, r in enumerate(runs)]).astype(np.int32)
+    n = pexp.size
+    # which kernel: the bf16 one above 40 pairs an expert, below it the thin one, whose blocks
+    # halve at 4 pairs an expert
+    assert (n > 40 * E) == (runs is DENSE_RUNS) and (n <= 4 * E) == (max(runs) <= 17)
+    res = []
+    for layer in (lay, _bf16_copy(lay)):
+        print(f"[bf16 order] {layer.spec.quant.mode} H={spec.hidden} I={spec.inter} pairs={n}", flush=True)
+        _, _, pool, _ = build_gpu_layer(layer, gpu)
+        pool.g2s_device(torch.cuda.current_stream().cuda_stream)
+        pool.device.sync()
+        y = torch.full((n, spec.hidden), float("nan"), dtype=torch.bfloat16, device=gpu)
+        dev = lambda a: torch.from_numpy(np.ascontiguousarray(a)).to(gpu)   # noqa: E731
+        ops.forward_pairs(layer.spec, pool, xd, dev(ptok), dev(pexp), dev(np.arange(n, dtype=np.int32)), y,
+                          L.FWD_FORCE_PREFILL)
+        torch.cuda.synchronize()
+        res.append(bits(y))
+        pool.close()
+    assert not np.isnan(F.bf16_bits_to_f32(res[0])).any()
+    assert np.array_equal(*res), f"{int((res[0] != res[1]).any(-1).sum())} of {n} rows differ"
