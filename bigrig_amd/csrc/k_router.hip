@@ -17,6 +17,7 @@ namespace {
 
 constexpr int kRouterThreads = 256;
 constexpr int kSmallT = 64;  // up to this many tokens: one wave per (row, 4 tokens) (5 us at 64); above: MFMA tiles (9 us)
+constexpr int kWideH = 5120;  // wider rows: see small_call
 
 // ---------------------------------------------------------------- many tokens
 // k_router_mfma: a block computes the logits of 16 M tokens x 16 M experts on fp32 MFMAs, in the
@@ -214,7 +215,7 @@ hipError_t mfma_launch(const brx_layer_desc& d, const void* x, const void* w_rou
 // ---------------------------------------------------------------- small T
 // k_router_logits: one wave per (expert row, tile of TT tokens), WPB waves per block; every
 // load of the wave is issued before the first FMA. Same per-lane chain and butterfly as
-// k_router, so the logits are the same bits.
+// k_router_mfma's, so the logits are the same bits.
 template <bool WF32, int TT, int WPB>
 __global__ __launch_bounds__(WPB * kWave) void k_router_logits(
     const uint16_t* __restrict__ x, const void* __restrict__ w, const float* __restrict__ bias,
@@ -381,6 +382,24 @@ hipError_t topk_launch(const brx_layer_desc& d, int T, int has_sg, const float* 
     return hipGetLastError();
 }
 
+// Calls that take one wave per (row, 4 tokens). Above kWideH inputs those of a few tiles do so past
+// kSmallT tokens too: a tile's K loop is then longer than the waves take, and this is the kernel those
+// calls had before the tiles. Waves / tiles, us, at 6144 inputs (5184 and 8192 move both alike; narrower
+// rows had a slower kernel than either before the tiles):
+//   to 128 tokens   bf16 8 experts x 100 9.2 / 19.7, 128 x 128 17.1 / 20.1, 256 x 80 20.4 / 20.5; fp32
+//                   128 x 100 20.2 / 21.5, 256 x 80 23.4 / 27.1; past the line 256 x 100 28.7 / 27.6
+//   to 256          bf16 64 x 256 16.2 / 20.0; fp32 32 x 256 13.9 / 21.3; past 128 x 180 21.9 / 20.4
+//   to 512          bf16 16 x 512 14.4 / 20.0; fp32 8 x 512 17.7 / 21.5; past 64 x 512 30.5 / 20.2
+//   to 1024         4 x 1024 15.0 / 20.0; past 8 x 1024 20.9 / 20.1
+bool small_call(const brx_layer_desc& d, int T) {
+    if (T <= kSmallT) return true;
+    if (d.hidden <= kWideH) return false;
+    const bool f32 = d.router_dtype == BRX_DT_F32;
+    const int rows_tokens = T <= 128 ? 20480 : T <= 256 ? (f32 ? 12800 : 16640) : T <= 512 ? (f32 ? 8192 : 16640)
+                          : T <= 1024 ? 4096 : 0;
+    return (int64_t)d.n_experts * T <= rows_tokens;
+}
+
 }  // namespace
 
 size_t router_workspace_bytes(const brx_layer_desc& d, int T) {
@@ -400,7 +419,7 @@ hipError_t launch_router(const brx_layer_desc& d, const void* x, const void* w_r
                          const float* bias, const void* sgw, int T, int32_t* out_idx,
                          float* out_w, float* out_sg, float* ws_logits, hipStream_t s) {
     if (T <= 0) return hipSuccess;
-    if (T <= kSmallT) {
+    if (small_call(d, T)) {
         hipError_t e = launch_router_logits(d, x, w_router, bias, sgw, T, ws_logits, s);
         if (e != hipSuccess) return e;
         return topk_launch(d, T, sgw ? 1 : 0, ws_logits, nullptr, nullptr, bias, out_idx, out_w, out_sg, s);

@@ -1,4 +1,5 @@
-"""The MFMA router (more than 64 tokens) ranks every expert as the oracle does, whatever the widths:
+"""The router for more than 64 tokens (MFMA tiles; rows of more than 5120 inputs with few experts and
+tokens a wave each) ranks every expert as the oracle does, whatever the widths:
 partial token and expert tiles, rows that end inside a 512-wide block of lane chains, bf16 and fp32
 router weights, a shared gate beside them. top_k is the expert count (at most 64), so the
 indices are the order of all logits: any logit off by a bit that changes the order of two shows."""
@@ -17,7 +18,8 @@ pytestmark = pytest.mark.gpu
 
 @pytest.mark.parametrize("f32", [False, True], ids=["bf16", "f32"])
 @pytest.mark.parametrize("T,H,E", [(65, 64, 16), (80, 512, 15), (81, 576, 17), (129, 1024, 64), (300, 2880, 33),
-                                   (97, 8192, 40), (2051, 192, 1),
+                                   (97, 8192, 40), (2051, 192, 1), (300, 8192, 64), (129, 5184, 128),
+                                  (513, 5184, 9), (512, 5184, 16),
                                    (2100, 576, 64), (1050, 1088, 257)])
 def test_full_ranking_matches_oracle(gpu, T, H, E, f32):
     base = E256_SHARED if E == 33 else OLMOE_1B_7B
