@@ -861,12 +861,25 @@ struct PfWs {
 
 inline size_t align256(size_t v) { return (v + 255) & ~(size_t)255; }
 
-// The M tile height of a kernel mode (kTileRows on the host; kDenseRows for bf16 weights), and the
-// height its smallest scratch is counted with (what brx_moe_block_forward_noalloc accepts).
-inline int tile_rows(int mode) {
-    return mode == kModeBf16 ? kDenseRows : mode == kModeAffine6 || mode == kModeAffine8 ? 64 : kBM;
+// The M tile height of a call the thin-tile GEMM does not take: kTileRows on the host; for bf16 weights
+// kDenseRows, or half of it while the blocks of the lower tiles (at most) are one round of the chip, one
+// a CU: taller tiles then only leave CUs idle. 256 / 128 rows, us a layer: 8 experts of 2048 x 768,
+// top-8, 160 tokens 103 / 74, 256 tokens 105 / 74; 4 experts of 4096 x 1024, top-2, 400 tokens 162 / 112;
+// past the line the 8 experts at 600 tokens 110 / 130, at 1000 117 / 142.
+inline int tile_rows(const FwdArgs& a) {
+    const int mode = a.quant_mode;
+    if (mode != kModeBf16) return mode == kModeAffine6 || mode == kModeAffine8 ? 64 : kBM;
+    const int64_t P_ext = a.P + (a.auto_shared ? a.T : 0), E_ext = a.E + (a.shared ? 1 : 0);
+    const int Imax = a.I > a.I_sh ? a.I : a.I_sh;
+    const int fpb = a.act == BRX_ACT_SILU_MLP ? kBlockN : kBlockN / 2;
+    const int nt_h = (Imax + fpb - 1) / fpb, nt_y = (a.H + kBlockN - 1) / kBlockN;
+    const int64_t tiles = (P_ext + kDenseRows / 2 - 1) / (kDenseRows / 2) + E_ext;
+    return tiles * (nt_h > nt_y ? nt_h : nt_y) <= kCus ? kDenseRows / 2 : kDenseRows;
 }
-inline int scratch_rows(int mode) { return mode == kModeBf16 ? 64 : tile_rows(mode); }
+// The height a call's smallest scratch is counted with (what brx_moe_block_forward_noalloc accepts): for
+// bf16 weights the 64 rows of the general kernel, which took them first, so what a scratch holds
+// is the same; the longer list covers both heights above.
+inline int scratch_rows(const FwdArgs& a) { return a.quant_mode == kModeBf16 ? 64 : tile_rows(a); }
 
 PfWs carve(const FwdArgs& a, int tile, void* ws) {
     const int P = a.P;
@@ -943,8 +956,8 @@ static int thin_rows(const FwdArgs& a) {
     return a.T <= 16 ? 16 : a.T <= 32 ? 32 : 64;
 }
 
-// What launch_prefill cannot do without, and what it takes when it may choose.
-size_t prefill_workspace_min(const FwdArgs& a) { return carve(a, scratch_rows(a.quant_mode), nullptr).bytes; }
+// What launch_prefill is sure to work in, and what it takes when it may choose.
+size_t prefill_workspace_min(const FwdArgs& a) { return carve(a, scratch_rows(a), nullptr).bytes; }
 
 size_t prefill_workspace_bytes(const FwdArgs& a) {
     const size_t m = prefill_workspace_min(a);
@@ -973,12 +986,13 @@ hipError_t launch_combine(const uint16_t* y_routed, const uint16_t* y_shared, co
 
 hipError_t launch_prefill(const FwdArgs& a, void* ws, size_t ws_bytes, int phases, hipStream_t s) {
     // (the lower tiles' longer list must fit a fixed scratch too; else the taller ones serve)
-    int tile = thin_rows(a);
-    PfWs w = carve(a, tile ? tile : tile_rows(a.quant_mode), ws);
-    if (tile && w.bytes > ws_bytes) {
-        tile = 0;
-        w = carve(a, tile_rows(a.quant_mode), ws);
+    int thin = thin_rows(a);
+    PfWs w = carve(a, thin ? thin : tile_rows(a), ws);
+    if (thin && w.bytes > ws_bytes) {
+        thin = 0;
+        w = carve(a, tile_rows(a), ws);
     }
+    const int tile = thin ? thin : tile_rows(a);
     if (w.bytes > ws_bytes) return hipErrorInvalidValue;
     const int P = a.P;
     const int T_sh = a.auto_shared ? a.T : 0;
@@ -990,13 +1004,13 @@ hipError_t launch_prefill(const FwdArgs& a, void* ws, size_t ws_bytes, int phase
     uint16_t* y_routed = a.yun ? a.yun : w.y_routed;
     hipError_t err = hipSuccess;
     if (phases & 1) {
-        err = launch_bucket(a.pexp, P, a.E, E_ext, T_sh, tile ? tile : tile_rows(a.quant_mode), a.g2s, a.capacity, a.host != nullptr, a.err, w.order, w.offsets,
-                            w.tile_start, w.tinfo, s);
+        err = launch_bucket(a.pexp, P, a.E, E_ext, T_sh, tile, a.g2s, a.capacity, a.host != nullptr, a.err, w.order,
+                            w.offsets, w.tile_start, w.tinfo, s);
         if (err != hipSuccess) return err;
     }
 #define BRX_GEMM(M) (a.scale_f16 ? launch_gemm<M, true>(a, w, E_ext, Imax, y_routed, phases, s) \
                                  : launch_gemm<M, false>(a, w, E_ext, Imax, y_routed, phases, s))
-    if (tile) {
+    if (thin) {
         err = launch_thin(a, ThinArgs{w.order, w.tile_start, w.tinfo, w.hbuf, y_routed, w.y_shared, E_ext, Imax,
                                       w.mt_pad, tile}, phases, s);
     } else switch (a.quant_mode) {
@@ -1008,7 +1022,7 @@ hipError_t launch_prefill(const FwdArgs& a, void* ws, size_t ws_bytes, int phase
         case BRX_QUANT_MXFP4: err = launch_gemm<BRX_QUANT_MXFP4, false>(a, w, E_ext, Imax, y_routed, phases, s); break;
         case kModeBf16:
             err = launch_dense(a, ThinArgs{w.order, w.tile_start, w.tinfo, w.hbuf, y_routed, w.y_shared, E_ext, Imax,
-                                           w.mt_pad, kDenseRows}, phases, s);
+                                           w.mt_pad, tile}, phases, s);
             break;
         default: err = hipErrorInvalidValue;
     }

@@ -6,7 +6,8 @@
 
 namespace brx {
 
-constexpr int kDenseRows = 256;   // pairs of an M tile of bf16 experts (k_dense.hip)
+constexpr int kCus = 256;
+constexpr int kDenseRows = 256;   // pairs of the tallest M tile of bf16 experts (k_dense.hip)
 
 // What the thin-tile and bf16 GEMMs take from the prefill launcher beside the forward's arguments.
 struct ThinArgs {

@@ -176,13 +176,14 @@ def _bf16_copy(lay):
     return replace(lay, spec=wide, experts=[conv(e) for e in lay.experts])
 
 
-DENSE_RUNS = [300, 256, 257, 129, 128, 127, 65, 64, 33, 32, 31, 1, 0, 7, 100, 200]   # tiles of 32 to 256 rows
+TALL_RUNS = [700, 513, 512, 511, 300, 257, 256, 255, 129, 128, 127, 65, 64, 33, 0, 1] + 112 * [25]   # to 256 rows
+DENSE_RUNS = [300, 256, 257, 129, 128, 127, 65, 64, 33, 32, 31, 1, 0, 7, 100, 200]                  # to 128 rows
 THIN_RUNS = [1, 15, 16, 17, 31, 32, 33, 63, 64, 65, 100, 0, 2, 7, 0, 3]               # 64-row tiles, 128-row blocks
 FEW_RUNS = [1, 15, 16, 17, 2, 0, 3, 0, 1, 0, 0, 2, 0, 0, 0, 1]                        # 64-row blocks
 
 
-@pytest.mark.parametrize("runs", [DENSE_RUNS, THIN_RUNS, FEW_RUNS, [min(r, 16) for r in FEW_RUNS]],
-                         ids=["dense", "thin", "thin-few", "thin-few16"])
+@pytest.mark.parametrize("runs", [TALL_RUNS, DENSE_RUNS, THIN_RUNS, FEW_RUNS, [min(r, 16) for r in FEW_RUNS]],
+                         ids=["tall", "dense", "thin", "thin-few", "thin-few16"])
 @pytest.mark.parametrize("kw", [dict(hidden=1536, inter=768), dict(hidden=576, inter=192, has_bias=True,
                                                                  act="swiglu_clamped"),
                                 dict(hidden=64, inter=64), dict(hidden=320, inter=448, act="silu_mlp")],
@@ -193,15 +194,19 @@ def test_bf16_rows_are_the_exactly_quantized_rows(gpu, kw, runs):
     import torch
     E = len(runs)
     spec = small(QWEN3_30B_A3B, n_experts=E, top_k=2, quant=F.QuantSpec(4, 32, "mxfp4"), **kw)
-    lay = make_layer(spec, seed=890)
+    lay = make_layer(spec, seed=890, bank=16)
     T = min(max(runs), 64)
     xd = to_dev_bits(make_x(T, spec.hidden, seed=891), gpu)
     pexp = np.repeat(np.arange(E, dtype=np.int32), runs)
     ptok = np.concatenate([(np.arange(r) * 3 + e) % T for e, r in enumerate(runs)]).astype(np.int32)
     n = pexp.size
-    # which kernel: the bf16 one above 40 pairs an expert, below it the thin one, whose blocks
-    # halve at 4 pairs an expert
-    assert (n > 40 * E) == (runs is DENSE_RUNS) and (n <= 4 * E) == (max(runs) <= 17)
+    # which kernel: the bf16 one above 40 pairs an expert, with 256-row tiles once those of 128 rows
+    # may be more than one block a CU; below it the thin one, whose blocks halve at 4 pairs an expert
+    assert (n > 40 * E) == (max(runs) > 100) and (n <= 4 * E) == (max(runs) <= 17)
+    if n > 40 * E and spec.hidden > 64:
+        fpb = 256 if spec.act == "silu_mlp" else 128
+        blocks = (-(-n // 128) + E) * max(-(-spec.inter // fpb), -(-spec.hidden // 256))
+        assert (blocks > 256) == (runs is TALL_RUNS)
     res = []
     for layer in (lay, _bf16_copy(lay)):
         print(f"[bf16 order] {layer.spec.quant.mode} H={spec.hidden} I={spec.inter} pairs={n}", flush=True)
