@@ -1636,6 +1636,28 @@ constexpr int kMaxUpl = MODE == kModeBf16 ? 2 : 4;
         }                                                                        \
     } while (0)
 
+// The weights of a projection over the step's possible entries (entries x H x I) from which a step of
+// several tokens runs per entry. Up to there the two launches saved matter more; from 32 entries on the
+// per-entry form wins at any width (8 tokens, top-4, 1024 x 512: 32.0 / 25.7 us a layer in three / five
+// launches). Replayed layers, three / five launches, us a layer:
+//   4-bit       4 entries 4096 x 1536 27.7 / 28.2, 4096 x 2048 30.3 / 31.7, 2 entries 4096 x 4096 29.8 / 31.9;
+//               3 and 4 entries 4096 x 4096 46.5 / 40.2 and 54.7 / 48.4; 3 entries 2880 x 2880 (three units a
+//               lane, which the one-launch kernel holds badly) 35.5 / 29.9; 6 and 10 entries
+//               2048 x 2048 28.4 / 27.9 and 41.3 / 36.3, 16 entries 2048 x 768 31.4 / 28.8
+//   2, 3 bits   as 4 bits; 6 and 8 bits and bf16 win per entry throughout (8 bits, 4 entries 4096 x 2048
+//               43.0 / 42.4)
+//   MXFP4       (little to dequantize, so the launches weigh more) 2 tokens: 4 entries 2880 x 2880 25.5 / 27.5,
+//               8192 x 2048 43.7 / 45.6, 4096 x 4096 40.7 / 39.6; 3 entries, 3 tokens 2880 x 2880 25.2 / 26.4,
+//               4096 x 4096 36.5 / 33.9; 8 entries 2048 x 2048 25.9 / 27.3, 4096 x 1536 36.3 / 34.5; 16 entries
+//               2048 x 1024 27.7 / 28.2, 2048 x 2048 45.4 / 39.2; 18 entries 1536 x 1024 28.6 / 27.0
+template <int MODE>
+int64_t per_entry_line(int T, int nu, int upl) {
+    int64_t m = 20;
+    if (MODE == BRX_QUANT_MXFP4) m = nu >= 18 ? 20 : nu > 4 ? 36 : T == 2 ? 70 : 40;
+    else if (kBits<MODE> <= 4 && nu <= 4 && T <= 3 && upl != 3) m = 35;
+    return m * 1000 * 1000;
+}
+
 template <int MODE>
 hipError_t launch_mode(const FwdArgs& a, uint16_t* hbuf, DecTable* table, uint16_t* y_routed,
                        uint16_t* y_shared, int phases, hipStream_t s) {
@@ -1643,16 +1665,6 @@ hipError_t launch_mode(const FwdArgs& a, uint16_t* hbuf, DecTable* table, uint16
     const int PT = P + (a.auto_shared ? a.T : 0);
     const int nu = P + (a.auto_shared ? 1 : 0);
     const int Imax = a.I > a.I_sh ? a.I : a.I_sh;
-    // Several tokens: either the plan launch, one block per (entry, rows) for each projection and the
-    // combine (five launches with the router), or one launch in which every gate/up block ranks and
-    // plans the step itself and a down kernel that stages every pair's h rows and combines (three).
-    // The first wins with many entries or much to multiply, the second where the two launches
-    // saved matter more. Three / five launches, us a layer: 2 tokens (16 entries) at H x I 2048 x 512
-    // 23.8 / 26.3, 2048 x 768 31.9 / 29.6; 3 tokens (24) at 1024 x 768 25.5 / 26.0, 2048 x 512 30.6 / 29.4,
-    // 2048 x 1024 49.2 / 42.4; 4 tokens (32) at 768 x 512 29.2 / 27.9, 2048 x 768 47.9 / 35.2; top-4 MXFP4 at
-    // 4 tokens (16) 1024 x 768 20.2 / 22.3, 2880 x 2880 95.6 / 58, at 8 tokens (32) 768 x 512 28.9 / 24.5 and
-    // 2880 x 2880 186 / 88. So the line: 32 entries, or 20 M weights a projection over the entries.
-    const bool per_entry = a.T > 1 && (nu >= 2 * kEntryRows || (int64_t)nu * a.H * Imax >= 20 * 1000 * 1000);
     // one token: one unit per lane where the row allows it (twice the waves of two units per
     // lane, each with half the dequant-dot work and far fewer registers: 11.1 -> 10.2 us per
     // layer on H = 2048); several tokens: two units per lane, half the blocks, each staging
@@ -1661,6 +1673,10 @@ hipError_t launch_mode(const FwdArgs& a, uint16_t* hbuf, DecTable* table, uint16
     // pairs share its launch (a pool's span calls against the whole step).
     int SPg, uplg;
     pick_split(a.H / 64, a.T > 1 && kMaxUpl<MODE> > 2 ? 2 : 1, SPg, uplg, kMaxUpl<MODE>);
+    // Several tokens: either the plan launch, one block per (entry, rows) for each projection and the
+    // combine (five launches with the router), or one launch in which every gate/up block ranks and
+    // plans the step itself and a down kernel that stages every pair's h rows and combines (three).
+    const bool per_entry = a.T > 1 && (nu >= 2 * kEntryRows || (int64_t)nu * a.H * Imax >= per_entry_line<MODE>(a.T, nu, uplg));
     // the one-token gate/up kernel makes every pair its own entry (pairs given by the caller may
     // repeat an expert, which the other kernels merge into one entry)
     const bool one_token = a.T == 1 && !a.ptok && uplg <= 3 && a.E <= 256 && nu <= kWave;
