@@ -73,10 +73,16 @@ def test_block_forward_refuses_a_pool_that_is_not_fully_resident(gpu, capacity):
     pool.close()
 
 
-@pytest.mark.parametrize("T", [2, 40], ids=["decode", "prefill"])
-def test_absent_expert_is_reported_and_its_rows_are_nan(gpu, T):
+# (10 pairs an expert and fewer: the thin-tile GEMM, in blocks of 64 weight rows up to 4; above 40 the
+# general one, or that of bf16 experts)
+@pytest.mark.parametrize("quant,T", [
+    (F.QuantSpec(4, 64, "affine"), 2), (F.QuantSpec(4, 64, "affine"), 40), (F.QuantSpec(6, 64, "affine"), 20),
+    (F.QuantSpec(8, 64, "affine"), 60), (F.QuantSpec(4, 32, "mxfp4"), 20), (F.QuantSpec(16, 0, "none"), 60),
+    (F.QuantSpec(8, 64, "affine"), 400), (F.QuantSpec(16, 0, "none"), 400)],
+    ids=["decode", "prefill", "thin-6bit", "thin-8bit", "thin-mxfp4", "thin-bf16", "general-8bit", "dense-bf16"])
+def test_absent_expert_is_reported_and_its_rows_are_nan(gpu, quant, T):
     import torch
-    spec = small(QWEN3_30B_A3B, hidden=512, inter=256, n_experts=32, top_k=4)
+    spec = small(QWEN3_30B_A3B, hidden=512, inter=256, n_experts=32, top_k=4, quant=quant)
     lay = make_layer(spec, seed=402)
     pool = _bounded(lay, 16, range(16))
     rng = np.random.default_rng(T)
@@ -86,7 +92,7 @@ def test_absent_expert_is_reported_and_its_rows_are_nan(gpu, T):
     x = make_x(T, spec.hidden, seed=4020 + T)
     out = torch.zeros((T, spec.hidden), dtype=torch.bfloat16, device=gpu)
     y = torch.zeros((T, spec.top_k, spec.hidden), dtype=torch.bfloat16, device=gpu)
-    print(f"[abi] absent expert T={T}", flush=True)
+    print(f"[abi] absent expert {quant.mode} {quant.bits}-bit T={T}", flush=True)
     ops.moe_forward(spec, pool, to_dev_bits(x, gpu), to_dev_bits(idx, gpu), to_dev_bits(w, gpu),
                     out=out, y_unreduced=y)
     lib = L.load()

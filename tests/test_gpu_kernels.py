@@ -110,17 +110,24 @@ def test_decode_layer(gpu, spec, T):
     pool.close()
 
 
-@pytest.mark.parametrize("spec", [small(QWEN3_30B_A3B, hidden=512, inter=768, n_experts=64, top_k=8),
-                                  small(GPT_OSS_120B, hidden=512, inter=1536, n_experts=32, top_k=4)],
-                         ids=["affine-I768", "mxfp4-I1536"])
-def test_decode_layer_staged_in_batches(gpu, spec):
-    """8 tokens whose h rows do not all fit in LDS: the down kernel stages them entry batch by
-    entry batch."""
+@pytest.mark.parametrize("spec,T,batches", [
+    (small(QWEN3_30B_A3B, hidden=256, inter=1536, n_experts=32, top_k=10), 3, True),
+    (small(GPT_OSS_120B, hidden=256, inter=1536, n_experts=32, top_k=10), 3, True),
+    (small(QWEN3_30B_A3B, hidden=256, inter=4096, n_experts=32, top_k=16), 1, True),
+    (small(GPT_OSS_120B, hidden=256, inter=4096, n_experts=32, top_k=16), 1, True),
+    (small(QWEN3_30B_A3B, hidden=512, inter=768, n_experts=64, top_k=8), 8, False),
+    (small(GPT_OSS_120B, hidden=512, inter=1536, n_experts=32, top_k=4), 8, False)],
+    ids=["affine-3tok", "mxfp4-3tok", "affine-1tok", "mxfp4-1tok", "affine-I768", "mxfp4-I1536"])
+def test_decode_layer_staged_in_batches(gpu, spec, T, batches):
+    """Steps whose h rows do not all fit in LDS: with one token, or few entries of few weights, the
+    down kernel stages them entry batch by entry batch; from 32 entries on one block an entry and
+    row block stages that entry's."""
     lay = make_layer(spec, seed=17, bank=8)
     moe, sw, pool, _ = build_gpu_layer(lay, gpu)
-    pairs = 8 * spec.top_k
+    pairs = T * spec.top_k
     assert pairs * (spec.inter // 64) * 148 > 96 * 1024
-    _layer_check(lay, moe, 8, seed=170, check_f64=False)
+    assert batches == (T == 1 or (pairs < 32 and pairs * spec.hidden * spec.inter < 20e6))
+    _layer_check(lay, moe, T, seed=170, check_f64=False)
     pool.close()
 
 

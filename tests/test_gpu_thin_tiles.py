@@ -1,9 +1,10 @@
 """Rows of the thin-tile GEMM equal the general grouped GEMM's, bit for bit.
 
-A call of at most 40 pairs an expert goes to the thin-tile kernel (M tiles of 16, 32 or 64 rows,
-blocks of 64 or 128 weight rows), a larger one to the general kernel, with the same operands in the
-same order: a row must have the same bits from both. The experts hold run lengths at the edges of
-the thin tiles; the same pairs repeated sixteen times take the general kernel. Widths give odd and
+A call of at most 40 pairs an expert goes to the thin-tile kernel (M tiles of 16, 32 or 64 rows;
+blocks of 64 weight rows up to 4 pairs an expert, of 128 above), a larger one to the general kernel
+(bf16: to its own), with the same operands in the same order: a row must have the same bits from
+both. The experts hold run lengths at the edges of the thin tiles; the same pairs repeated sixteen
+times take the general kernel. Widths give odd and
 single 64-wide stages and last column blocks that are half empty.
 """
 import numpy as np
@@ -20,6 +21,9 @@ from tests.helpers import make_layer, make_x, small
 pytestmark = pytest.mark.gpu
 
 RUNS = [1, 15, 16, 17, 31, 32, 33, 63, 64, 65, 100, 0, 2, 7, 0, 3]   # pairs of expert 0, 1, ...
+FEW64 = [40, 1, 0, 2, 16, 0, 0, 3, 0, 0, 0, 0, 0, 0, 0, 1]
+FEW32 = [1, 2, 0, 15, 16, 17, 0, 3, 0, 0, 4, 0, 2, 0, 0, 1]
+FEW16 = [1, 2, 0, 8, 16, 7, 0, 3, 0, 0, 4, 0, 2, 0, 0, 1]
 Q = F.QuantSpec
 
 
@@ -27,8 +31,11 @@ def _spec(H, I, quant, **kw):
     return small(QWEN3_30B_A3B, hidden=H, inter=I, n_experts=len(RUNS), top_k=2, quant=quant, **kw)
 
 
-@pytest.mark.parametrize("runs", [RUNS, [min(r, 32) for r in RUNS], [min(r, 16) for r in RUNS]],
-                         ids=["rows64", "rows32", "rows16"])
+# (runs, weight rows of a block without and with the shared expert's pairs)
+@pytest.mark.parametrize("runs,block,block_shared", [
+    (RUNS, 128, 128), ([min(r, 32) for r in RUNS], 128, 128), ([min(r, 16) for r in RUNS], 128, 128),
+    (FEW64, 64, 128), (FEW32, 64, 128), (FEW16, 64, 64)],
+    ids=["rows64", "rows32", "rows16", "few64", "few32", "few16"])
 @pytest.mark.parametrize("spec", [
     _spec(512, 256, Q(4, 64, "affine")),
     _spec(576, 320, Q(4, 64, "affine", "float16")),
@@ -45,7 +52,7 @@ def _spec(H, I, quant, **kw):
     small(E256_SHARED, hidden=512, inter=192, n_experts=len(RUNS), top_k=4, shared_inter=320),
 ], ids=["4bit", "4bit-f16-odd", "4bit-one-stage", "4bit-g128", "3bit-odd", "2bit-odd", "2bit-g128", "6bit-odd",
         "8bit-odd", "mxfp4-odd", "bf16-odd", "silu-mlp", "shared"])
-def test_thin_rows_equal_general_rows(gpu, spec, runs):
+def test_thin_rows_equal_general_rows(gpu, spec, runs, block, block_shared):
     import torch
     T = max(runs)        # 16, 32 or more tokens: the thin tile heights
     lay = make_layer(spec, seed=41)
@@ -73,7 +80,9 @@ def test_thin_rows_equal_general_rows(gpu, spec, runs):
         torch.cuda.synchronize()
         return bits(y)
 
-    assert n <= 40 * spec.n_experts < 16 * n
+    E_ext = spec.n_experts + (1 if shared is not None else 0)
+    assert n <= 40 * E_ext < 16 * n
+    assert (n <= 4 * E_ext) == ((block_shared if spec.shared_inter else block) == 64)
     thin, general = run(1), run(16)
     for c in range(16):
         part = general[c * n:(c + 1) * n]

@@ -77,3 +77,35 @@ def test_noalloc_refuses_a_call_beyond_its_scratch(gpu):
     assert "scratch" in lib.brx_last_error().decode()
     assert bool((out.float() == 3.0).all()) and bool((idx == -1).all())
     pool.close()
+
+
+def _prefill_bytes(T, spec, rows):
+    """The bytes a prefill of T tokens carves with M tiles of `rows` rows: routing, then the lists, h and y."""
+    al = lambda v: -(-v // 256) * 256   # noqa: E731
+    E, P = spec.n_experts, T * spec.top_k
+    tiles = -(-(-(-P // rows) + E) // 8) * 8
+    return (al(4 * T * (E + 1)) + 2 * al(4 * P) + al(4 * P) + 2 * al(4 * (E + 1)) + al(16 * tiles) +
+            al(2 * P * spec.inter) + al(2 * P * spec.hidden))
+
+
+def test_noalloc_takes_taller_tiles_where_the_thin_list_does_not_fit(gpu):
+    """A call that the no-alloc scratch holds with 128-row tiles and not with the 64-row ones its few
+    pairs an expert would take: accepted, with the bits of the call over the grown workspace."""
+    import torch
+    lib = L.load()
+    spec = small(QWEN3_30B_A3B, hidden=64, inter=832, n_experts=256, top_k=4)
+    T = 2034
+    assert T * spec.top_k <= 40 * spec.n_experts
+    assert _prefill_bytes(T, spec, 128) <= L.NOALLOC_SCRATCH_BYTES < _prefill_bytes(T, spec, 64)
+    lay = make_layer(spec, seed=503, bank=8, zipf=0.5)
+    moe, sw, pool, _ = build_gpu_layer(lay, gpu)
+    pool.g2s_device(torch.cuda.current_stream().cuda_stream)
+    print(f"[noalloc] thin list past the scratch T={T}", flush=True)
+    args = (spec, pool, to_dev_bits(make_x(T, spec.hidden, seed=5030), gpu), to_dev_bits(lay.router, gpu),
+            to_dev_bits(lay.bias, gpu), None, None, 0)
+    rc0, out0, idx0, w0 = _call(lib.brx_moe_block_forward, *args)
+    rc1, out1, idx1, w1 = _call(lib.brx_moe_block_forward_noalloc, *args)
+    assert rc0 == 0 and rc1 == 0, lib.brx_last_error().decode()
+    assert np.array_equal(idx1.cpu().numpy(), idx0.cpu().numpy())
+    assert np.array_equal(bits(out1), bits(out0))
+    pool.close()
