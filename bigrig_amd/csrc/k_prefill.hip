@@ -948,11 +948,16 @@ hipError_t launch_bucket(const int32_t* pexp, int P, int E, int E_ext, int T_sh,
 // The M tile height of a call whose tiles all go to the thin-tile GEMM (k_thin.hip), or 0 for
 // k_pf_gemm. The line is the mean number of pairs an expert: both kernels within 2% at 48 (777
 // tokens of 128 3-bit experts, 179 against 176 us), the thin one faster at 32 (512 tokens of 4-bit
-// experts, two layers: 272 against 290 us) and below.
+// experts, two layers: 272 against 290 us) and below. A pool with host backing may have every tile read
+// its expert's weights over the bus, where one tile more costs what it copies: past 64 tokens such a call
+// takes the tallest tiles of its format (32 of 128 experts resident, Zipf routing, 4-bit, 128 / 256 / 512
+// tokens: 2.52 / 3.34 / 5.36 ms in 64-row tiles, 2.36 / 3.12 / 4.43 in 128-row ones; up to 64 tokens no expert
+// has more than one tile).
 static int thin_rows(const FwdArgs& a) {
     constexpr int kThinPairs = 40;
     const int64_t P_ext = a.P + (a.auto_shared ? a.T : 0), E_ext = a.E + (a.shared ? 1 : 0);
     if (P_ext > kThinPairs * E_ext) return 0;
+    if (a.host && a.T > 64 && tile_rows(a) > 64) return 0;
     return a.T <= 16 ? 16 : a.T <= 32 ? 32 : 64;
 }
 
