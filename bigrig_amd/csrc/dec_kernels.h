@@ -1373,8 +1373,8 @@ __global__ __launch_bounds__(kThreads) void k_dec_down(FwdArgs a, const uint16_t
     dec_down_epilogue(a, ys, RBD, lrbd, n0);
 }
 
-// The down kernel when the h rows of every pair fit in LDS (every decode step of the shipped
-// shapes): each row group reads its item's table row itself, the h rows are staged by pair id,
+// The down kernel of one token, and of several in one launch, when the h rows of every pair fit in
+// LDS: each row group reads its item's table row itself, the h rows are staged by pair id,
 // and the item's weights are requested as soon as its slot is known -- two memory round trips
 // in all, no scan and one barrier before the dot products.
 template <int MODE, int UPL, int NT>

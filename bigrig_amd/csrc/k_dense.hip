@@ -1,7 +1,7 @@
 // Grouped GEMM of unquantized bf16 experts (chunks; batches and short chunks go to k_thin.hip).
 //
-// One block = 8 waves, one block a CU; tile = 256, 128, 64 or 32 of an expert's pairs x 256 weight
-// rows (KIND 0: the gate and up rows of 128 features). Wave (wm, wn) owns 32 MR pairs and 64 weight
+// One block = 8 waves, one block a CU; tile = 256, 128, 64 or 32 of an expert's pairs (the tallest a call
+// cuts: tile_rows in k_prefill.hip) x 256 weight rows (KIND 0: the gate and up rows of 128 features). Wave (wm, wn) owns 32 MR pairs and 64 weight
 // rows, so at MR 4 a 16-K step reads 4 A and 2 B fragments from LDS for 8 v_mfma_f32_32x32x16_bf16
 // (96 of the 128 bytes a clock LDS gives at the full MFMA rate). There is nothing to dequantize, so
 // both operands are copied straight into LDS by the buffer unit in 64-K stages: whole 128-byte lines

@@ -9,9 +9,10 @@
 //   k_bucket   one block per expert: in one pass over the pairs, the histogram of all of them
 //              and the stable (pair-order) compaction of the expert's pairs into LDS; then the
 //              expert's run offset, the run copied out in order, and one tile descriptor {expert,
-//              first bucketed row, rows, slot} per 128-row M tile, placed in a tile list that
-//              holds every tile of more than 64 rows before the smaller ones, so the GEMM grids
-//              dispatch the long tiles first and the short ones fill the end.
+//              first bucketed row, rows, slot} per M tile of up to BM rows (16 to 256, by the GEMM
+//              the call takes), placed in a tile list that holds every tile of more than BM / 2
+//              rows before the smaller ones, so the GEMM grids dispatch the long tiles first and
+//              the short ones fill the end.
 //   k_pf_gemm  grouped GEMM, tile = (M tile of one expert's pairs, 256 columns), one wave
 //              per SIMD, v_mfma_f32_32x32x16_bf16.  KIND 0 (gate/up): A rows are the pairs'
 //              token activations gathered from x, B rows the gate and up weights of 128
